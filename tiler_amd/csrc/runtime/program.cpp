@@ -1286,6 +1286,28 @@ tiler_hip_status plan_expression(const Target& t, uint32_t dtype, uint64_t n, co
 
 // ---------------------------------------------------------------------------
 // Serial folds over any reduced-axis set.  Slots: x, out, [epilogue program].
+// Whether the reduced axes longer than 1 are adjacent (axes of extent 1 move
+// nothing): the tensor is then [outer, reduced, inner] with the contributors
+// in ascending order along the middle axis.
+static bool adjacent_axes(uint32_t rank, const uint64_t* dims, uint64_t reduced_mask, uint64_t& outer,
+                          uint64_t& inner) {
+  outer = inner = 1;
+  bool reduced = false, after = false;
+  for (uint32_t d = 0; d < rank; ++d) {
+    if (dims[d] == 1) continue;
+    if (reduced_mask >> d & 1) {
+      if (after) return false;
+      reduced = true;
+    } else if (reduced) {
+      after = true;
+      inner *= dims[d];
+    } else {
+      outer *= dims[d];
+    }
+  }
+  return reduced;
+}
+
 tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uint64_t reduced_mask,
                            uint32_t scale_bits, uint32_t bias_bits, const ExpressionProgram* epilogue,
                            Program& p, const Contract& c, const Target* t, const tiler_hip_sum_plan* sp,
@@ -1389,6 +1411,49 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
   float scale, bias;
   std::memcpy(&scale, &scale_bits, 4);
   std::memcpy(&bias, &bias_bits, 4);
+  uint64_t outer, inner;
+  if (t && addr && !epilogue && contributors >= 16 &&
+      adjacent_axes(rank, dims, reduced_mask, outer, inner)) {
+    // The reduced axes are adjacent: [outer, contributors, inner].
+    char name[48];
+    const uint64_t cus = t->compute_units;
+    if (inner == 1 && outputs <= 0x7fffffffull) {
+      // contiguous rows: the staged strict sums (a prologue as a rule under
+      // the preserving modes), or the maximum's row kernel
+      if (op == TILER_HIP_FOLD_SUM) {
+        add_serial_fold(*t, x, aligned16(addr[x]), outputs, contributors, out, p);
+        return TILER_HIP_OK;
+      }
+      if (op != TILER_HIP_FOLD_MAXIMUM) {
+        FoldRuleHost rule;
+        rule.prologue = op == TILER_HIP_FOLD_SQUARED ? 1u : 2u;
+        rule.scale = scale;
+        rule.bias = bias;
+        add_rule_fold(*t, x, aligned16(addr[x]), outputs, contributors, out, rule, p);
+        return TILER_HIP_OK;
+      }
+      // 16 lanes to a row, a wave, or a workgroup for long or few rows
+      const uint32_t lanes = contributors >= 2048 || outputs <= 4 * cus ? 256 : contributors > 256 ? 64 : 16;
+      const uint32_t per = 256 / lanes;
+      p.add("tiler_fold_maximum_f32_rows", (uint32_t)((outputs + per - 1) / per), 1, 256)
+          .ptr(x).ptr(out).u64(outputs).u64(contributors).u32(lanes);
+      return TILER_HIP_OK;
+    }
+    const uint64_t groups = mul_sat(outer, (inner + 15) / 16), blocks = (outputs + 255) / 256;
+    // A workgroup per 16 columns up to one wave of outputs per CU, where a
+    // lane per output waits on its own loads (sum, cols against lanes, us:
+    // 1 x 4096 x 4096 18.6 / 102, 16 x 1024 x 1024 22 / 31); above that the
+    // lanes alone fill memory (1000 x 256 x 64 24 / 12.7, 64 x 64 x 4096
+    // 81 / 11.8), and short folds do not fill a stage (300 x 50 x 1000
+    // 97 / 11.7).  The columns' 32-bit offsets take inner below 2^21.
+    const bool cols = contributors >= 128 && outputs <= 64 * cus && inner < (1ull << 21);
+    if (inner > 1 && (cols ? groups : blocks) <= 0x7fffffffull) {
+      std::snprintf(name, sizeof(name), "%s_%s", kNames[op], cols ? "cols" : "lanes");
+      p.add(name, (uint32_t)(cols ? groups : blocks), 1, !cols ? 256 : op == TILER_HIP_FOLD_MAXIMUM ? 512 : 576)
+          .ptr(x).ptr(out).u64(cols ? groups : outputs).u64(contributors).u64(inner).f32(scale).f32(bias);
+      return TILER_HIP_OK;
+    }
+  }
   Launch& l = p.add(kNames[op], blocks_capped(outputs, 65536), 1, 256)
                   .ptr(x).ptr(out).u64(outputs).u64(contributors).blob(&g, sizeof(g), 8)
                   .f32(scale).f32(bias).u32(0);

@@ -283,6 +283,15 @@ const EntryRow kEntries[] = {
     {"tiler_fold_squared_f32", "squared-serial-sum-f32/serial", 3},
     {"tiler_fold_fma_f32", "fused-multiply-add-serial-sum-f32/serial", 3},
     {"tiler_fold_maximum_f32", "strict-serial-maximum-f32/serial", 3},
+    {"tiler_fold_sum_f32_lanes", "strict-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_sum_f32_cols", "strict-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_squared_f32_lanes", "squared-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_squared_f32_cols", "squared-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_fma_f32_lanes", "fused-multiply-add-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_fma_f32_cols", "fused-multiply-add-serial-sum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_maximum_f32_lanes", "strict-serial-maximum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_maximum_f32_cols", "strict-serial-maximum-f32/serial-adjacent-axes", 2},
+    {"tiler_fold_maximum_f32_rows", "strict-serial-maximum-f32/serial-rows", 2},
 #define TILER_EXPR_ROWS(TY, FAM)                                                                  \
   {"tiler_expr_" TY "_r16_i0", FAM, 18}, {"tiler_expr_" TY "_r16_i1", FAM, 18},                     \
       {"tiler_expr_" TY "_r16_i2", FAM, 18}, {"tiler_expr_" TY "_r16_i3", FAM, 18},                 \
@@ -1819,7 +1828,10 @@ tiler_hip_status tiler_hip_fold_f32(tiler_hip_context* ctx, uint32_t variant, co
                                     uint32_t bias_bits, float* out, tiler_hip_stream stream) try {
   if (!ctx) return TILER_HIP_REFUSE_INVALID_ARGUMENT;
   tiler_rt::Program p;
-  tiler_hip_status st = tiler_rt::plan_fold(variant, rank, dims, reduced_mask, scale_bits, bias_bits, nullptr, p);
+  const uintptr_t addr[2] = {(uintptr_t)x, (uintptr_t)out};
+  const tiler_rt::Target target = target_of(ctx);
+  tiler_hip_status st = tiler_rt::plan_fold(variant, rank, dims, reduced_mask, scale_bits, bias_bits, nullptr, p,
+                                            tiler_rt::Contract{}, &target, nullptr, addr);
   if (st != TILER_HIP_OK) return fail(ctx, st, p.diag);
   if (p.nlaunches && (!x || !out)) return TILER_HIP_REFUSE_INVALID_ARGUMENT;
   void* slots[tiler_rt::kMaxSlots] = {const_cast<float*>(x), out};
