@@ -11,5 +11,6 @@
 #include "fold.hip"
 #include "convert.hip"
 #include "contract.hip"
+#include "contract_ksplit.hip"
 #include "contract_general.hip"
 #include "dequantize.hip"

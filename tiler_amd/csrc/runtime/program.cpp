@@ -783,6 +783,62 @@ tiler_hip_status plan_contract_strict_f32(const Target& t, uint64_t m, uint64_t 
   return TILER_HIP_OK;
 }
 
+// The k-split tiles (contract_ksplit.hip): MB x NB blocks of 16 x 16 outputs,
+// W waves.
+struct KsplitTile {
+  uint32_t mb, nb, waves;
+};
+static const KsplitTile kKsplitTiles[] = {{2, 2, 8}, {4, 2, 8}, {2, 4, 8}, {3, 4, 8}, {4, 4, 4},
+                                          {5, 4, 8}, {6, 4, 4}, {4, 8, 4}, {6, 8, 4}};
+
+bool is_ksplit(const char* symbol) {
+  const char* k = std::strstr(symbol, "_k");
+  return k && k[2] >= '1' && k[2] <= '9';
+}
+
+// Workgroups of a k-split launch per batch: the kernel takes panels of B in
+// groups of eight (one per XCD) where there are as many.
+static uint64_t ksplit_grid(uint64_t m, uint64_t n, uint32_t mb, uint32_t nb) {
+  const uint64_t tm = (m + 16 * mb - 1) / (16 * mb), tn = (n + 16 * nb - 1) / (16 * nb);
+  return mul_sat(tm, tn >= 8 ? (tn + 7) / 8 * 8 : tn);
+}
+
+// The k-split tile for `batches` products of m x n x k, or null where the
+// 128- or 256-tiles are the better form.  Times in ns, fitted on the device
+// over m 65..3000 and n, k 616..8192 (root mean square error 14%; the choice
+// costs 1% over the best of the tiles and the staged forms):
+// * k-split: 2400 + rounds of tiles over the CUs x (0.392 k (MB + NB), the
+//   operand fill, + 136 per block, the fold of the partial tiles); two
+//   workgroups of at most 80 KiB share a CU, so a part round costs them less;
+// * 128-tiles: 3400 + 660 per 64-deep k tile, 1050 with two tiles on a CU;
+//   twice that in the general form, which serves n off the 8-element grid.
+// A k-split tile has to be a tenth faster by these to be taken.  From k = 512
+// on each of eight waves has a chunk of its own.
+static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batches) {
+  if (k < 512 || k >= (1ull << 24)) return nullptr;
+  const uint64_t cus = t.compute_units;
+  const uint64_t t256 = mul_sat(mul_sat((m + 255) / 256, (n + 255) / 256), batches);
+  if (t256 >= cus) return nullptr;
+  const uint64_t t128 = mul_sat(mul_sat((m + 127) / 128, (n + 127) / 128), batches);
+  const uint64_t steps = (k + 63) / 64;
+  uint64_t staged = 3400 + (t128 <= cus ? 660 * steps : 1050 * steps * ((t128 + 2 * cus - 1) / (2 * cus)));
+  if (n % 8 != 0) staged *= 2;
+  const KsplitTile* best = nullptr;
+  uint64_t best_ns = staged * 9 / 10;
+  for (const KsplitTile& c : kKsplitTiles) {
+    const uint64_t tm = (m + 16 * c.mb - 1) / (16 * c.mb), tn = (n + 16 * c.nb - 1) / (16 * c.nb);
+    const uint64_t tiles = tm * tn * batches;  // t256 < cus bounds all three
+    uint64_t rounds = (tiles + cus - 1) / cus * 1000;  // in thousandths
+    if ((c.mb + c.nb) * c.waves <= 40) {
+      rounds = (660 * rounds + 340 * (tiles * 1000 / cus)) / 1000;
+      if (rounds < 1000) rounds = 1000;
+    }
+    const uint64_t ns = 2400 + rounds * (392 * k * (c.mb + c.nb) / 1000 + 136 * c.mb * c.nb) / 1000;
+    if (ns < best_ns) best_ns = ns, best = &c;
+  }
+  return best;
+}
+
 tiler_hip_status plan_contract_bf16(const Target& t, uint64_t m, uint64_t n, uint64_t k,
                                     uint32_t epilogue, const uintptr_t* addr, Program& p, bool strict,
                                     uint32_t form, bool live_k) {
@@ -837,11 +893,22 @@ tiler_hip_status plan_contract_bf16(const Target& t, uint64_t m, uint64_t n, uin
   if (form == TILER_HIP_FORM_CONTRACT_SKINNY && !skinny_ok)
     return p.refuse(TILER_HIP_REFUSE_UNSUPPORTED,
                     "skinny-rows: the skinny form takes m <= 64 and k a multiple of 8, aligned operands");
-  if (skinny_ok && (pick || form == TILER_HIP_FORM_CONTRACT_SKINNY)) {
+  // (k past 2^24: the general form, whose offsets are 64 bits)
+  if (skinny_ok && k < (1ull << 24) && (pick || form == TILER_HIP_FORM_CONTRACT_SKINNY)) {
+    const uint32_t mb = (uint32_t)((m + 15) / 16);
     char name[48];
-    std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u", silu ? "silu_" : "", (uint32_t)((m + 15) / 16));
-    p.add(name, (uint32_t)((n + 15) / 16), 1, 1024).ptr(a).ptr(b).u32(m32).u32(n32).u32(k32).ptr(c);
+    std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u", silu ? "silu_" : "", mb);
+    p.add(name, (uint32_t)ksplit_grid(m, n, mb, 1), 1, 512).ptr(a).ptr(b).u32(m32).u32(n32).u32(k32).ptr(c);
     return TILER_HIP_OK;
+  }
+  if (pick && m > 64 && k % 8 == 0 && aligned16(addr[a]) && aligned16(addr[b])) {
+    if (const KsplitTile* ks = ksplit_tile(t, m, n, k, 1)) {
+      char name[48];
+      std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sk%ux%u", silu ? "silu_" : "", ks->mb, ks->nb);
+      p.add(name, (uint32_t)ksplit_grid(m, n, ks->mb, ks->nb), 1, 64 * ks->waves)
+          .ptr(a).ptr(b).u32(m32).u32(n32).u32(k32).ptr(c);
+      return TILER_HIP_OK;
+    }
   }
   // The staged path addresses each operand panel (up to 256 rows) through one
   // buffer resource with 32-bit offsets (256 * k * 2 bytes must stay below
@@ -1040,9 +1107,15 @@ tiler_hip_status plan_contract_general(const Target& t, uint32_t dtype, const ti
       const uint32_t m32 = (uint32_t)m, n32 = (uint32_t)n, k32 = (uint32_t)k;
       const bool ab_al = aligned16(addr[l]) && (right_kn || aligned16(addr[r])) && strides8;
       char name[48];
-      if (m <= 64 && k % 8 == 0 && ab_al) {
-        std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u_b", silu ? "silu_" : "", (uint32_t)((m + 15) / 16));
-        p.add(name, (uint32_t)((n + 15) / 16), (uint32_t)batches, 1024)
+      const KsplitTile* ks = nullptr;
+      if (k % 8 == 0 && k < (1ull << 24) && ab_al) {
+        static const KsplitTile kSkinny[] = {{1, 1, 8}, {2, 1, 8}, {3, 1, 8}, {4, 1, 8}};
+        ks = m <= 64 ? &kSkinny[(m - 1) / 16] : ksplit_tile(t, m, n, k, batches);
+      }
+      if (ks) {
+        if (m <= 64) std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u_b", silu ? "silu_" : "", ks->mb);
+        else std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sk%ux%u_b", silu ? "silu_" : "", ks->mb, ks->nb);
+        p.add(name, (uint32_t)ksplit_grid(m, n, ks->mb, ks->nb), (uint32_t)batches, 64 * ks->waves)
             .ptr(l).ptr(right_slot).u32(m32).u32(n32).u32(k32).ptr(o).blob(&g, sizeof g, 8);
         return TILER_HIP_OK;
       }

@@ -209,6 +209,9 @@ tiler_hip_status plan_contract_bf16(const Target& t, uint64_t m, uint64_t n, uin
                                     uint32_t epilogue, const uintptr_t* addr, Program& p,
                                     bool strict = false, uint32_t form = TILER_HIP_FORM_AUTO,
                                     bool live_k = false);
+// Whether `symbol` is one of the k-split contraction tiles beyond m = 64
+// (tiler_contract_bf16_[silu_]k{MB}x{NB}).
+bool is_ksplit(const char* symbol);
 // Pointwise expression over n elements: slots inputs 0..I-1, y, program
 // (CONSTANT), and -- for programs beyond the register form -- the value
 // store (SCRATCH).  `addr` covers the inputs then y.

@@ -327,6 +327,13 @@ const EntryRow kEntries[] = {
     {"tiler_contract_bf16_silu_t128_kf", "tensor-contraction-bf16/cooperative+silu", 3},
     {"tiler_contract_bf16_t256_kf", "tensor-contraction-bf16/cooperative", 3},
     {"tiler_contract_bf16_silu_t256_kf", "tensor-contraction-bf16/cooperative+silu", 3},
+#define TILER_KSPLIT_ROWS(K)                                                       \
+  {"tiler_contract_bf16_" K, "tensor-contraction-bf16/cooperative", 3},             \
+      {"tiler_contract_bf16_silu_" K, "tensor-contraction-bf16/cooperative+silu", 3}
+    TILER_KSPLIT_ROWS("k2x2"), TILER_KSPLIT_ROWS("k4x2"), TILER_KSPLIT_ROWS("k2x4"), TILER_KSPLIT_ROWS("k3x4"),
+    TILER_KSPLIT_ROWS("k4x4"), TILER_KSPLIT_ROWS("k5x4"), TILER_KSPLIT_ROWS("k6x4"), TILER_KSPLIT_ROWS("k4x8"),
+    TILER_KSPLIT_ROWS("k6x8"),
+#undef TILER_KSPLIT_ROWS
     // general index structures: the strict fold (geometry in a constant slot),
     // the batched MFMA forms and the right-operand transpose ahead of them
     {"tiler_contract_general_f32", "tensor-contraction-f32/strict-general", 4},
@@ -338,7 +345,9 @@ const EntryRow kEntries[] = {
       {"tiler_contract_bf16_silu_" K "_b", "tensor-contraction-bf16/cooperative-batched+silu", 3}
     TILER_BATCHED_ROWS("t256"), TILER_BATCHED_ROWS("t128"), TILER_BATCHED_ROWS("skinny1"),
     TILER_BATCHED_ROWS("skinny2"), TILER_BATCHED_ROWS("skinny3"), TILER_BATCHED_ROWS("skinny4"),
-    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"),
+    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"), TILER_BATCHED_ROWS("k2x2"), TILER_BATCHED_ROWS("k4x2"),
+    TILER_BATCHED_ROWS("k2x4"), TILER_BATCHED_ROWS("k3x4"), TILER_BATCHED_ROWS("k4x4"), TILER_BATCHED_ROWS("k5x4"),
+    TILER_BATCHED_ROWS("k6x4"), TILER_BATCHED_ROWS("k4x8"), TILER_BATCHED_ROWS("k6x8"),
 #undef TILER_BATCHED_ROWS
 };
 constexpr uint32_t kEntryCount = sizeof(kEntries) / sizeof(kEntries[0]);
@@ -2485,11 +2494,17 @@ tiler_hip_status tiler_hip_propose(const tiler_hip_context* ctx, const tiler_hip
       } forms[] = {{"gfx950.contraction.mfma-skinny", TILER_HIP_FORM_CONTRACT_SKINNY},
                    {"gfx950.contraction.mfma-staged-256", TILER_HIP_FORM_CONTRACT_STAGED_256},
                    {"gfx950.contraction.mfma-staged-128", TILER_HIP_FORM_CONTRACT_STAGED_128},
-                   {"gfx950.contraction.mfma-general-128", TILER_HIP_FORM_CONTRACT_GENERAL_128}};
+                   {"gfx950.contraction.mfma-general-128", TILER_HIP_FORM_CONTRACT_GENERAL_128},
+                   {"gfx950.contraction.mfma-k-split", TILER_HIP_FORM_AUTO}};
       tiler_rt::Program autop;
       const bool auto_ok = reassociate && plan_region(ctx, &base, autop) == TILER_HIP_OK;
       chosen = s0;
       for (const auto& f : forms) {
+        // the k-split tiles are offered where they are the library's own choice
+        // (the shapes that leave the staged tiles' chip idle)
+        if (f.form == TILER_HIP_FORM_AUTO &&
+            !(auto_ok && autop.nlaunches && tiler_rt::is_ksplit(autop.launches[0].symbol)))
+          continue;
         tiler_hip_region v = base;
         v.form = f.form;
         const uint64_t extent = f.form == TILER_HIP_FORM_CONTRACT_SKINNY ? e[0] : e[1] % 8 ? e[1] : e[2];
