@@ -16,7 +16,7 @@ RE = L.PERMITS_REASSOCIATION
 CASES = [
     (1, 16, 8, "skinny1"), (16, 17, 520, "skinny1"), (7, 130, 72, "skinny1"), (31, 100, 1000, "skinny2"),
     (33, 24, 512, "skinny3"), (64, 1001, 584, "skinny4"), (49, 136, 64, "skinny4"),
-    (65, 64, 512, "k2x2"), (97, 121, 1032, "k2x2"), (129, 2001, 520, "k4x2"), (66, 4100, 584, "k2x4"),
+    (65, 64, 512, "k2x2"), (97, 121, 1032, "k2x2"), (129, 2001, 520, "k2x4"), (66, 4100, 584, "k2x4"),
     (100, 4104, 520, "k3x4"), (500, 1999, 1000, "k4x4"), (201, 4100, 520, "k5x4"), (1300, 1001, 512, "k6x4"),
     (1000, 1999, 1000, "k4x8"), (490, 4100, 1032, "k6x8"),
 ]

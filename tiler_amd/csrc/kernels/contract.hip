@@ -169,15 +169,147 @@ __device__ __forceinline__ void contract_strict_blocked_body(const T* __restrict
   }
 }
 
+// A column per lane: a workgroup of W waves owns 64 columns and TM W rows, and
+// a wave TM rows of the tile.  The right operand's 64 rows go to LDS 64 steps
+// of k at a time (buffer_load ... lds, 16 bytes a lane where k is a multiple of
+// 4 and b 16-byte aligned, else 4), double-buffered, a lane reading four steps
+// of its own row per 16-byte read; chunk c of row r sits at c ^ (r & 15), so 16
+// lanes cover the banks.  The left operand's rows are the same for every lane
+// and come through the scalar cache: a product is one v_mul_f32 with a scalar
+// operand, so a step costs two VALU instructions per row, a quarter LDS read
+// and a share of a scalar load.  Operands of the next KB steps are requested
+// before the current ones are folded (the s_waitcnt at the head of a block
+// covers both kinds, which share a counter and return in any order).  The same
+// ascending first-product fold; steps past k are never folded, rows past m
+// read the last one and are not stored.
+//
+// Bound by VALU issue where the chip is full (512 x 3072 x 1024: 70 us, 46 T
+// operations/s; the register-blocked 32 x 32 tiles took 113), else by the
+// latency of a block's operands.  Before and now, us: 17 x 1024 x 1024
+// 29 / 10.2, 128 x 3072 x 1024 49 / 27, 128 x 1024 x 3072 90 / 34,
+// 256 x 1024 x 1024 44 / 17.6, 300 x 3000 x 2000 285 / 111.
+template <int TM, int KB, int W>
+__device__ __forceinline__ void contract_strict_columns_body(const float* __restrict__ a,
+                                                             const float* __restrict__ b, uint32_t m, uint32_t n,
+                                                             uint32_t k, float* __restrict__ c, uint32_t row0,
+                                                             uint32_t col0) {
+  typedef __attribute__((address_space(3))) void lds_ptr;
+  constexpr int kBlk = 64 / KB;
+  constexpr int kLgkm0 = 0xC07F;  // lgkmcnt(0)
+  __shared__ __align__(1024) float stage[2 * 64 * 64];
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t cols = n - col0 < 64u ? n - col0 : 64u;
+  const __amdgpu_buffer_rsrc_t pb =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(b + (uint64_t)col0 * k), (short)0, cols * k * 4u, 0x00020000);
+  const bool wide = (k & 3u) == 0 && ((uintptr_t)b & 15u) == 0;
+  auto issue = [&](uint32_t s) {
+    float* dst = stage + (s & 1u) * 4096u;
+    if (wide) {
+#pragma unroll
+      for (uint32_t j = 0; j < 16 / W; ++j) {
+        const uint32_t q = wave * (16 / W) + j, row = q * 4u + (lane >> 4);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(pb, (lds_ptr*)(dst + q * 256u), 16,
+                                                 row * k * 4u + s * 256u + ((lane & 15u) ^ (row & 15u)) * 16u, 0, 0, 0);
+      }
+    } else {
+#pragma unroll 4
+      for (uint32_t j = 0; j < 64 / W; ++j) {
+        const uint32_t row = wave * (64 / W) + j;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            pb, (lds_ptr*)(dst + row * 64u), 4,
+            row * k * 4u + s * 256u + (((lane >> 2) ^ (row & 15u)) * 4u + (lane & 3u)) * 4u, 0, 0, 0);
+      }
+    }
+  };
+  const float* ar[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const uint32_t r = row0 + wave * TM + i;
+    ar[i] = a + (uint64_t)(r < m ? r : m - 1u) * k;
+  }
+  float av[2][TM][KB];
+  f32x4 bv[2][KB / 4];
+  auto load_a = [&](float (&v)[TM][KB], uint32_t at) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < KB; ++e) v[i][e] = ar[i][at + e];
+  };
+  auto load_b = [&](f32x4 (&v)[KB / 4], const float* src, uint32_t kb) {
+#pragma unroll
+    for (int q = 0; q < KB / 4; ++q)
+      v[q] = *reinterpret_cast<const f32x4*>(src + (((kb * (KB / 4) + q) ^ (lane & 15u)) << 2));
+  };
+  float acc[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) acc[i] = -0.0f;  // -0 + first product == first product
+  const uint32_t stages = (k + 63u) / 64u, whole = k / 64u;
+  issue(0);
+  if (whole) load_a(av[0], 0);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (uint32_t s = 0; s < whole; ++s) {
+    if (s + 1 < stages) issue(s + 1);  // into the buffer every wave left at the last barrier
+    const float* src = stage + (s & 1u) * 4096u + lane * 64u;
+    load_b(bv[0], src, 0);
+    const uint32_t next = s + 1 < whole ? (s + 1) * 64u : 0u;
+    auto block = [&](auto kbs) -> bool {
+      constexpr int kb = decltype(kbs)::value, p = kb & 1;
+      __builtin_amdgcn_s_waitcnt(kLgkm0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kb + 1 < kBlk) {
+        load_a(av[p ^ 1], s * 64u + (kb + 1) * KB);
+        load_b(bv[p ^ 1], src, kb + 1);
+      } else {
+        load_a(av[p ^ 1], next);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < KB; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i] = acc[i] + av[p][i][e] * bv[p][e / 4][e % 4];
+      __builtin_amdgcn_sched_barrier(0);
+      return true;
+    };
+    tiler::unrolled_while<0, kBlk>(block);
+    // this wave's share of stage s + 1 has landed; its reads of stage s were
+    // waited for at the head of the last block
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  if (whole < stages) {
+    const float* src = stage + (whole & 1u) * 4096u + lane * 64u;
+    const uint32_t count = k - whole * 64u;
+    for (uint32_t e = 0; e < count; ++e) {
+      const float bw = src[(((e >> 2) ^ (lane & 15u)) << 2) + (e & 3u)];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[i] = acc[i] + ar[i][whole * 64u + e] * bw;
+    }
+  }
+  if (lane < cols) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const uint32_t r = row0 + wave * TM + i;
+      if (r < m) c[(uint64_t)r * n + col0 + lane] = canon(acc[i]);
+    }
+  }
+}
+
+// Tiles of 4 rows (b16: as many outputs as a 16 x 16 tile) and of 16 (b32).
+// The column tiles are the fast index, so those of one XCD (workgroup id % 8)
+// repeat over the rows and its L2 keeps their panels; blockIdx.x also counts
+// the 4 (2) row tiles of each 16 (32) rows.
 extern "C" __global__ void __launch_bounds__(256)
 tiler_contract_strict_f32_b16(const float* __restrict__ a, const float* __restrict__ b, uint32_t m, uint32_t n,
                               uint32_t k, float* __restrict__ c) {
-  contract_strict_blocked_body<1, 1>(a, b, m, n, k, c);
+  const uint32_t tiles_n = (n + 63u) / 64u, row0 = blockIdx.y * 16u + blockIdx.x / tiles_n * 4u;
+  if (row0 >= m) return;
+  contract_strict_columns_body<1, 32, 4>(a, b, m, n, k, c, row0, blockIdx.x % tiles_n * 64u);
 }
-extern "C" __global__ void __launch_bounds__(256)
+extern "C" __global__ void __launch_bounds__(512)
 tiler_contract_strict_f32_b32(const float* __restrict__ a, const float* __restrict__ b, uint32_t m, uint32_t n,
                               uint32_t k, float* __restrict__ c) {
-  contract_strict_blocked_body<2, 2>(a, b, m, n, k, c);
+  const uint32_t tiles_n = (n + 63u) / 64u, row0 = blockIdx.y * 32u + blockIdx.x / tiles_n * 16u;
+  if (row0 >= m) return;
+  contract_strict_columns_body<2, 8, 8>(a, b, m, n, k, c, row0, blockIdx.x % tiles_n * 64u);
 }
 #define TILER_CONTRACT_STRICT_BF16_BLOCKED(EDGE, T)                                                    \
   extern "C" __global__ void __launch_bounds__(256)                                                    \

@@ -214,7 +214,6 @@ TILER_CONTRACT_KSPLIT_BOTH(skinny2, 2, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(skinny3, 3, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(skinny4, 4, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k2x2, 2, 2, 8)
-TILER_CONTRACT_KSPLIT_BOTH(k4x2, 4, 2, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k2x4, 2, 4, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k3x4, 3, 4, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k4x4, 4, 4, 4)

@@ -716,7 +716,7 @@ static void declare_live_k(Program& p, uint64_t bound) {
   p.nlive = 1;
 }
 
-// Register-blocked strict tiles of 16·T x 16·T, T x T outputs per thread,
+// Register-blocked strict bf16 tiles of 16·T x 16·T, T x T outputs per thread,
 // T in {1, 2, 4}: the one with the least work on the busiest CU -- rounds of
 // tiles over the CUs x outputs per tile x the time per output step, relative
 // weights 31 : 20 : 18 (T = 1 measured 1.4-1.7 x T = 2 per output step on the
@@ -734,6 +734,26 @@ static uint32_t strict_tile(const Target& t, uint64_t m, uint64_t n) {
     if (cost < best_cost) best_cost = cost, best = T;
   }
   return best;
+}
+
+// The strict f32 forms for k >= 64: a column per lane with 4 or 16 rows to a
+// workgroup of 64 columns, or the register-blocked 64 x 64 tiles.
+// * 4 rows while that is at most four workgroups per CU: more waves to hide
+//   the operands' latency (256 x 1024 x 1024, 1024 of them: 19.8 us against
+//   25.9 with twice the rows; 128 x 3072 x 1024, 1536: 30.3 against 26.5).
+// * Then 16 rows or the 64 x 64 tiles, by the work on the busiest CU: rounds x
+//   outputs per workgroup x a weight in quarter units, measured per output
+//   step (1024 x 3072 x 1024, three rounds of 64 x 64: 160 against 179 us;
+//   2048 x 2048 x 1024, four: 218 against 212).
+// * The column forms address a tile's 64 rows of k with 32-bit offsets.
+enum class StrictForm { kRows4, kRows16, kTile64 };
+static StrictForm strict_f32_form(const Target& t, uint64_t m, uint64_t n, uint64_t k) {
+  const uint64_t cus = t.compute_units, tn = (n + 63) / 64;
+  if (k >= (1ull << 24)) return StrictForm::kTile64;
+  if (mul_sat(tn, (m + 3) / 4) <= 4 * cus) return StrictForm::kRows4;
+  const uint64_t r16 = (mul_sat(tn, (m + 15) / 16) + cus - 1) / cus;
+  const uint64_t r64 = (mul_sat(tn, (m + 63) / 64) + cus - 1) / cus;
+  return mul_sat(r16, 1024 * 76) <= mul_sat(r64, 4096 * 72) + 4096 * 12 ? StrictForm::kRows16 : StrictForm::kTile64;
 }
 
 tiler_hip_status plan_contract_strict_f32(const Target& t, uint64_t m, uint64_t n, uint64_t k, const uintptr_t* addr,
@@ -766,11 +786,13 @@ tiler_hip_status plan_contract_strict_f32(const Target& t, uint64_t m, uint64_t 
     return TILER_HIP_OK;
   }
   if (k >= 64) {
-    const uint32_t best = strict_tile(t, m, n);
-    const uint32_t tile = 16 * best;
-    static const char* const names[] = {nullptr, "tiler_contract_strict_f32_b16", "tiler_contract_strict_f32_b32",
-                                        nullptr, "tiler_contract_strict_f32_b64"};
-    Launch& l = p.add(names[best], (uint32_t)((n + tile - 1) / tile), (uint32_t)((m + tile - 1) / tile), 256)
+    const StrictForm f = strict_f32_form(t, m, n, k);
+    const uint64_t tn = (n + 63) / 64;
+    const uint32_t gx = (uint32_t)(f == StrictForm::kRows4 ? 4 * tn : f == StrictForm::kRows16 ? 2 * tn : tn);
+    const uint32_t edge = f == StrictForm::kRows4 ? 16 : f == StrictForm::kRows16 ? 32 : 64;
+    char name[40];
+    std::snprintf(name, sizeof(name), "tiler_contract_strict_f32_b%u", edge);
+    Launch& l = p.add(name, gx, (uint32_t)((m + edge - 1) / edge), f == StrictForm::kRows16 ? 512 : 256)
                     .ptr(a).ptr(b).u32((uint32_t)m).u32((uint32_t)n);
     (live_k ? l.live_u32(0) : l.u32((uint32_t)k)).ptr(c);
     return TILER_HIP_OK;
@@ -788,7 +810,7 @@ tiler_hip_status plan_contract_strict_f32(const Target& t, uint64_t m, uint64_t 
 struct KsplitTile {
   uint32_t mb, nb, waves;
 };
-static const KsplitTile kKsplitTiles[] = {{2, 2, 8}, {4, 2, 8}, {2, 4, 8}, {3, 4, 8}, {4, 4, 4},
+static const KsplitTile kKsplitTiles[] = {{2, 2, 8}, {2, 4, 8}, {3, 4, 8}, {4, 4, 4},
                                           {5, 4, 8}, {6, 4, 4}, {4, 8, 4}, {6, 8, 4}};
 
 bool is_ksplit(const char* symbol) {

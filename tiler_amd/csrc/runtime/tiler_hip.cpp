@@ -330,7 +330,7 @@ const EntryRow kEntries[] = {
 #define TILER_KSPLIT_ROWS(K)                                                       \
   {"tiler_contract_bf16_" K, "tensor-contraction-bf16/cooperative", 3},             \
       {"tiler_contract_bf16_silu_" K, "tensor-contraction-bf16/cooperative+silu", 3}
-    TILER_KSPLIT_ROWS("k2x2"), TILER_KSPLIT_ROWS("k4x2"), TILER_KSPLIT_ROWS("k2x4"), TILER_KSPLIT_ROWS("k3x4"),
+    TILER_KSPLIT_ROWS("k2x2"), TILER_KSPLIT_ROWS("k2x4"), TILER_KSPLIT_ROWS("k3x4"),
     TILER_KSPLIT_ROWS("k4x4"), TILER_KSPLIT_ROWS("k5x4"), TILER_KSPLIT_ROWS("k6x4"), TILER_KSPLIT_ROWS("k4x8"),
     TILER_KSPLIT_ROWS("k6x8"),
 #undef TILER_KSPLIT_ROWS
@@ -345,8 +345,7 @@ const EntryRow kEntries[] = {
       {"tiler_contract_bf16_silu_" K "_b", "tensor-contraction-bf16/cooperative-batched+silu", 3}
     TILER_BATCHED_ROWS("t256"), TILER_BATCHED_ROWS("t128"), TILER_BATCHED_ROWS("skinny1"),
     TILER_BATCHED_ROWS("skinny2"), TILER_BATCHED_ROWS("skinny3"), TILER_BATCHED_ROWS("skinny4"),
-    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"), TILER_BATCHED_ROWS("k2x2"), TILER_BATCHED_ROWS("k4x2"),
-    TILER_BATCHED_ROWS("k2x4"), TILER_BATCHED_ROWS("k3x4"), TILER_BATCHED_ROWS("k4x4"), TILER_BATCHED_ROWS("k5x4"),
+    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"), TILER_BATCHED_ROWS("k2x2"), TILER_BATCHED_ROWS("k2x4"), TILER_BATCHED_ROWS("k3x4"), TILER_BATCHED_ROWS("k4x4"), TILER_BATCHED_ROWS("k5x4"),
     TILER_BATCHED_ROWS("k6x4"), TILER_BATCHED_ROWS("k4x8"), TILER_BATCHED_ROWS("k6x8"),
 #undef TILER_BATCHED_ROWS
 };
