@@ -88,6 +88,35 @@ __device__ __forceinline__ float fold_combine(const FoldRule& r, float acc, floa
   return canon(subnormal(r.out_mode, subnormal(r.in_mode, acc) + subnormal(r.in_mode, t)));
 }
 
+// The wave reads subnormal binary32 operands as the zero of their sign and
+// keeps subnormal results (FP32 denorm field of MODE = 2): the sign-preserving
+// input mode in hardware, on every operand of every multiply and add, exactly
+// (the result side is left alone on purpose: the hardware decides to flush a
+// product before it is rounded, the reference after).  A fold whose result
+// mode flushes with the sign needs nothing more inside its chain, since every
+// result is read next as a flushed operand: only its last result is flushed,
+// by flush_sign.  Called before the first load, so no arithmetic precedes it.
+__device__ __forceinline__ void flush_operands_in_hardware() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), 2" ::: "memory");
+}
+// A subnormal to the zero of its sign, by integer operations (no mode applies).
+__device__ __forceinline__ float flush_sign(float v) {
+  const uint32_t b = __float_as_uint(v);
+  return __uint_as_float((b & 0x7f800000u) == 0 ? b & 0x80000000u : b);
+}
+// Whether a rule's modes are what flush_operands_in_hardware gives: the input
+// mode flushing with the sign, the result mode doing the same or preserving.
+__device__ __forceinline__ bool hardware_modes(const FoldRule& r) { return r.in_mode == 2u && r.out_mode != 3u; }
+// A contributor and a combine under them; canonical NaNs are left to the commit.
+__device__ __forceinline__ float fold_contributor_hw(const FoldRule& r, float v) {
+  if (r.prologue == kPrologueSquared) return v * v;
+  if (r.prologue == kPrologueFma) {
+    const float p = v * r.scale;
+    return p + r.bias;
+  }
+  return v;
+}
+
 // bf16 <-> f32 (ADR 0091 decision 2): widening is exact; narrowing is
 // round-to-nearest-even on the upper half, every NaN to 0x7fc0, signed zero
 // kept, gradual underflow, overflow to infinity at the inclusive midpoint.

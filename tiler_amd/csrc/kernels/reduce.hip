@@ -302,7 +302,7 @@ __device__ __forceinline__ void staged_relay_body(const float* __restrict__ x, u
 template <int R>
 constexpr uint32_t kRuleStageFloats = 2u * R * (4096u / R + 4u);  // both buffers of R rows
 
-template <int R, bool kVec, bool kIn, bool kOut>
+template <int R, bool kVec, bool kIn, bool kOut, bool kHw = false>
 __device__ __forceinline__ void staged_rule_body(const float* __restrict__ x, uint64_t nrows, uint64_t length,
                                                  float* __restrict__ out, const tiler::FoldRule& rule,
                                                  float* __restrict__ lds) {
@@ -323,6 +323,7 @@ __device__ __forceinline__ void staged_rule_body(const float* __restrict__ x, ui
     return __builtin_amdgcn_classf(v, 0x90) ? __uint_as_float(__float_as_uint(v) & mask) : v;
   };
   auto operand = [&](float v) {  // apply_to_operand(contributor(v))
+    if constexpr (kHw) return tiler::fold_contributor_hw(rule, v);  // the add that reads it flushes it
     const float c = tiler::fold_contributor(rule, v);
     return kIn ? flush(c, imask) : c;
   };
@@ -358,6 +359,10 @@ __device__ __forceinline__ void staged_rule_body(const float* __restrict__ x, ui
   float acc = 0.0f, acc_o = 0.0f;  // R's last result, and O of it
   auto step = [&](float to) {
     const float sum = acc_o + to;
+    if constexpr (kHw) {
+      acc = acc_o = sum;
+      return;
+    }
     acc = kOut ? flush(sum, rmask) : sum;
     acc_o = (kIn && !kOut) ? flush(acc, imask) : acc;
   };
@@ -390,7 +395,7 @@ __device__ __forceinline__ void staged_rule_body(const float* __restrict__ x, ui
     if (more) store((uint32_t)((s + 1) & 1));
     __syncthreads();
   }
-  if (folds) out[row0 + fr] = tiler::canon(acc);
+  if (folds) out[row0 + fr] = tiler::canon(kHw && kOut ? tiler::flush_sign(acc) : acc);
 }
 
 // R in {1, 4, 16}: the relay fold; R = 64 and 256 (rows of 16..255): the
@@ -427,7 +432,7 @@ TILER_SUM_STAGED(256, staged_lane_body)  // rows of 16..63: stages of 16 element
 // leaves the value unchanged (R(acc + -0.0) = R(acc) = acc for a value that
 // came out of R); with only the input mode flushing it would leave O(acc),
 // so there the row's last pass takes a step only below the row's end.
-template <int R, bool kVec, bool kIn, bool kOut>
+template <int R, bool kVec, bool kIn, bool kOut, bool kHw = false>
 __device__ __forceinline__ void staged_rule_relay_body(const float* __restrict__ x, uint64_t nrows, uint64_t length,
                                                        float* __restrict__ out, const tiler::FoldRule& rule,
                                                        float* __restrict__ lds) {
@@ -452,6 +457,7 @@ __device__ __forceinline__ void staged_rule_relay_body(const float* __restrict__
     return __builtin_amdgcn_classf(v, 0x90) ? __uint_as_float(__float_as_uint(v) & mask) : v;
   };
   auto operand = [&](float v) {  // apply_to_operand(contributor(v))
+    if constexpr (kHw) return tiler::fold_contributor_hw(rule, v);  // the add that reads it flushes it
     const float c = tiler::fold_contributor(rule, v);
     return kIn ? flush(c, imask) : c;
   };
@@ -486,6 +492,7 @@ __device__ __forceinline__ void staged_rule_relay_body(const float* __restrict__
   };
   // acc is R's last result; O(acc) is taken at the next step.
   auto step = [&](float acc, float to) {
+    if constexpr (kHw) return acc + to;
     const float acc_o = (kIn && !kOut) ? flush(acc, imask) : acc;
     const float sum = acc_o + to;
     return kOut ? flush(sum, rmask) : sum;
@@ -543,24 +550,33 @@ __device__ __forceinline__ void staged_rule_relay_body(const float* __restrict__
     if (more) store((uint32_t)((st + 1) & 1), st + 1);
     __syncthreads();
   }
-  if (folding_wave && s == 0 && g < kRowsPerWave && row0 + fr < nrows) out[row0 + fr] = tiler::canon(acc);
+  if (folding_wave && s == 0 && g < kRowsPerWave && row0 + fr < nrows)
+    out[row0 + fr] = tiler::canon(kHw && kOut ? tiler::flush_sign(acc) : acc);
 }
 
 // The same stages under a FoldRule: a flushing contract's serial fold, and the
 // fused prologues (squared, scale-bias) over a trailing axis; one body per
-// pair of flushing dimensions, chosen by a uniform branch.
+// pair of flushing dimensions, chosen by a uniform branch.  kHw: the modes the
+// hardware applies (flush_operands_in_hardware), which leaves the chain the
+// preserving fold's one add per element instead of an add, a class test and a
+// select: serial 1024 x 16384 under the flushing contract 243 -> 57 us.
 template <int R, bool kVec>
 __device__ __forceinline__ void staged_rule_dispatch(const float* __restrict__ x, uint64_t nrows, uint64_t length,
                                                      float* __restrict__ out, const tiler::FoldRule& rule) {
   __shared__ __align__(16) float lds[kRuleStageFloats<R>];
-  const bool in = rule.in_mode > 1u, res = rule.out_mode > 1u;
+  const bool in = rule.in_mode > 1u, res = rule.out_mode > 1u, hw = tiler::hardware_modes(rule);
+  if (hw) tiler::flush_operands_in_hardware();
   if constexpr (R <= 16) {  // the relay fold (rows of at least 256 elements per stage)
-    if (in && res) staged_rule_relay_body<R, kVec, true, true>(x, nrows, length, out, rule, lds);
+    if (hw && res) staged_rule_relay_body<R, kVec, true, true, true>(x, nrows, length, out, rule, lds);
+    else if (hw) staged_rule_relay_body<R, kVec, true, false, true>(x, nrows, length, out, rule, lds);
+    else if (in && res) staged_rule_relay_body<R, kVec, true, true>(x, nrows, length, out, rule, lds);
     else if (in) staged_rule_relay_body<R, kVec, true, false>(x, nrows, length, out, rule, lds);
     else if (res) staged_rule_relay_body<R, kVec, false, true>(x, nrows, length, out, rule, lds);
     else staged_rule_relay_body<R, kVec, false, false>(x, nrows, length, out, rule, lds);
   } else {
-    if (in && res) staged_rule_body<R, kVec, true, true>(x, nrows, length, out, rule, lds);
+    if (hw && res) staged_rule_body<R, kVec, true, true, true>(x, nrows, length, out, rule, lds);
+    else if (hw) staged_rule_body<R, kVec, true, false, true>(x, nrows, length, out, rule, lds);
+    else if (in && res) staged_rule_body<R, kVec, true, true>(x, nrows, length, out, rule, lds);
     else if (in) staged_rule_body<R, kVec, true, false>(x, nrows, length, out, rule, lds);
     else if (res) staged_rule_body<R, kVec, false, true>(x, nrows, length, out, rule, lds);
     else staged_rule_body<R, kVec, false, false>(x, nrows, length, out, rule, lds);
@@ -617,60 +633,189 @@ tiler_sum_f32_partials_m(const float* __restrict__ x, uint64_t rows, uint64_t ex
 
 // CooperativeWorkgroup: one workgroup per row; blockDim.x == participants.
 // Round r: participant p folds cell (RoundMajor r*P+p | ParticipantMajor p*R+r)
-// of `chunk` contributors; staged partials go to LDS; participant 0 folds them
-// in ascending p and accumulates round totals in ascending r -- the single
+// of `chunk` contributors; the partials go to LDS; participant 0 folds them in
+// ascending p and accumulates round totals in ascending r -- the single
 // workgroup tree of tiler-metal's cooperative_workgroup_reduction golden.
+//
+// A participant that folds its cell straight from global memory touches a line
+// per load that its neighbours do not share, and waits for each: 4096 x 4096
+// under the flushing contract took 80 us.  The workgroup instead stages S
+// elements of every cell at a time through LDS (S a power of two that keeps
+// the stage within kCoopFloats), neighbouring participants loading
+// neighbouring elements, and each folds its cell's run from there; the cells
+// lie S + 4 floats apart, so 16 lanes' 16-byte reads touch every bank once.
+// Stages of 20 KiB leave six workgroups to a CU to overlap one's loads with
+// another's fold: 19 us, 3.5 TB/s (1024 x 16384 98 -> 18.5 us).
+//
+// combine(acc, t) and contributor(v) are the rule's (evaluate.rs:845-1158
+// cooperative_grouped_sum_under: every cell, the partials and the round totals
+// seeded at their first value); kVec: 16-byte loads.
+constexpr uint32_t kCoopFloats = 5120;
+
+// The largest power of two S <= 64 with participants * (S + 4) floats in the
+// stage, at most the cell rounded up; below 4 (more than 640 participants) the
+// cells are folded straight from memory.
+__device__ __forceinline__ uint32_t coop_run(uint32_t participants, uint64_t chunk) {
+  const uint32_t room = kCoopFloats / participants;
+  uint32_t s = 64;
+  while (s >= 4 && (s + 4 > room || (s > 4 && s / 2 >= chunk))) s >>= 1;
+  return s;
+}
+
+template <bool kVec, typename C, typename F>
+__device__ __forceinline__ float coop_body(const float* __restrict__ row, uint32_t participants, uint64_t chunk,
+                                           uint64_t rounds, uint32_t participant_major, C contributor, F combine,
+                                           float* __restrict__ stage, uint32_t group, uint32_t cells) {
+  float* const staged = stage + kCoopFloats;
+  constexpr uint32_t W = kVec ? 4 : 1, kBatch = 8;
+  typedef typename std::conditional<kVec, f32x4, float>::type piece;
+  const uint32_t p = threadIdx.x;
+  const uint32_t S = coop_run(participants, chunk), pieces = S / W;
+  const uint32_t shift = 31u - __builtin_clz(pieces | 1u);
+  float total = 0.0f;
+  for (uint64_t r = 0; r < rounds; ++r) {
+    const uint64_t first = participant_major ? r * chunk : r * participants * chunk;       // cell of participant 0
+    const uint64_t apart = participant_major ? rounds * chunk : chunk;                      // between cells
+    float partial = 0.0f;
+    if (S >= 4) {
+      for (uint64_t e0 = 0; e0 < chunk; e0 += S) {
+        for (uint32_t i0 = 0; i0 < pieces; i0 += kBatch) {
+          piece v[kBatch];
+#pragma unroll
+          for (uint32_t i = 0; i < kBatch; ++i) {
+            const uint32_t id = (i0 + i) * participants + p, q = id >> shift, j = (id & (pieces - 1u)) * W;
+            v[i] = piece{};
+            if (i0 + i < pieces && q < cells && e0 + j < chunk) {
+              const float* src = row + first + q * apart + e0 + j;
+              if constexpr (kVec) v[i] = *reinterpret_cast<const f32x4*>(src);
+              else v[i] = *src;
+            }
+          }
+#pragma unroll
+          for (uint32_t i = 0; i < kBatch; ++i) {
+            const uint32_t id = (i0 + i) * participants + p, q = id >> shift, j = (id & (pieces - 1u)) * W;
+            if (i0 + i < pieces) *reinterpret_cast<piece*>(&stage[q * (S + 4u) + j]) = v[i];
+          }
+        }
+        __syncthreads();
+        const float* run = stage + p * (S + 4u);
+        const uint32_t count = chunk - e0 < S ? (uint32_t)(chunk - e0) : S;
+        uint32_t c = 0;
+        if (e0 == 0) {
+          partial = contributor(run[0]);
+          for (c = 1; c < 4 && c < count; ++c) partial = combine(partial, contributor(run[c]));
+        }
+#pragma unroll 4
+        for (; c + 4 <= count; c += 4) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(run + c);
+          partial = combine(partial, contributor(v.x));
+          partial = combine(partial, contributor(v.y));
+          partial = combine(partial, contributor(v.z));
+          partial = combine(partial, contributor(v.w));
+        }
+        for (; c < count; ++c) partial = combine(partial, contributor(run[c]));
+        __syncthreads();
+      }
+    } else {
+      const float* range = row + first + (p < cells ? p : 0u) * apart;
+      partial = contributor(range[0]);
+      for (uint64_t w = 1; w < chunk; ++w) partial = combine(partial, contributor(range[w]));
+    }
+    staged[p] = partial;
+    __syncthreads();
+    if (p % group == 0) {
+      const float* mine = staged + p;
+      float s = mine[0];
+      uint32_t q = 1;
+      for (; q < 4 && q < group; ++q) s = combine(s, mine[q]);
+      if ((group & 3u) == 0) {
+#pragma unroll 4
+        for (; q + 4 <= group; q += 4) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(mine + q);
+          s = combine(s, v.x);
+          s = combine(s, v.y);
+          s = combine(s, v.z);
+          s = combine(s, v.w);
+        }
+      }
+      for (; q < group; ++q) s = combine(s, mine[q]);
+      total = r == 0 ? s : combine(total, s);
+    }
+    __syncthreads();
+  }
+  return total;
+}
+// One row to a workgroup (kPacked false), or blockDim.x / participants rows of
+// one round: their cells lie end to end, so the workgroup stages them as one
+// run of cells, and the first participant of each row folds its partials.
+// Small groups are bound by the rate at which workgroups start: 65536 rows of
+// 16 participants took 116 us one to a workgroup and take 15 packed.
+template <bool kPacked, typename C, typename F>
+__device__ __forceinline__ void coop_rows(const float* __restrict__ x, uint64_t rows, uint64_t extent,
+                                          uint32_t participants, uint64_t chunk, uint64_t rounds,
+                                          uint32_t participant_major, float* __restrict__ out, bool flush,
+                                          C contributor, F combine, float* __restrict__ lds) {
+  const uint32_t per = kPacked ? blockDim.x / participants : 1u, threads = kPacked ? blockDim.x : participants;
+  const uint64_t row0 = (uint64_t)blockIdx.x * per;
+  const uint32_t live = kPacked && rows - row0 < per ? (uint32_t)(rows - row0) : per;
+  const float* row = x + row0 * extent;
+  float total;
+  if (((uintptr_t)x & 15u) == 0 && (chunk & 3u) == 0)  // uniform: every cell starts 16-byte aligned
+    total = coop_body<true>(row, threads, chunk, rounds, participant_major, contributor, combine, lds, participants,
+                            live * participants);
+  else
+    total = coop_body<false>(row, threads, chunk, rounds, participant_major, contributor, combine, lds, participants,
+                             live * participants);
+  const uint32_t g = threadIdx.x / participants;
+  if (threadIdx.x % participants == 0 && g < live)
+    out[row0 + g] = canon(flush ? tiler::flush_sign(total) : total);
+}
+template <bool kPacked>
+__device__ __forceinline__ void coop_rule_rows(const float* __restrict__ x, uint64_t rows, uint64_t extent,
+                                               uint32_t participants, uint64_t chunk, uint64_t rounds,
+                                               uint32_t participant_major, float* __restrict__ out,
+                                               const tiler::FoldRule& rule, float* __restrict__ lds) {
+  // (a lone contributor is transported, not read by an add: the general rule)
+  if (tiler::hardware_modes(rule) && extent > 1) {
+    tiler::flush_operands_in_hardware();
+    coop_rows<kPacked>(x, rows, extent, participants, chunk, rounds, participant_major, out, rule.out_mode > 1u,
+                       [&](float v) { return tiler::fold_contributor_hw(rule, v); },
+                       [](float acc, float t) { return acc + t; }, lds);
+  } else {
+    coop_rows<kPacked>(x, rows, extent, participants, chunk, rounds, participant_major, out, false,
+                       [&](float v) { return tiler::fold_contributor(rule, v); },
+                       [&](float acc, float t) { return tiler::fold_combine(rule, acc, t); }, lds);
+  }
+}
+
 extern "C" __global__ void __launch_bounds__(1024)
 tiler_sum_f32_cooperative(const float* __restrict__ x, uint64_t extent, uint32_t participants,
                           uint64_t chunk, uint64_t rounds, uint32_t participant_major,
                           float* __restrict__ out) {
-  __shared__ float staged[1024];
-  const uint32_t p = threadIdx.x;
-  const float* row = x + (uint64_t)blockIdx.x * extent;
-  float total = -0.0f;
-  for (uint64_t r = 0; r < rounds; ++r) {
-    uint64_t cell = participant_major ? (uint64_t)p * rounds + r : r * participants + p;
-    const float* range = row + cell * chunk;
-    float partial = -0.0f;
-    for (uint64_t w = 0; w < chunk; ++w) partial = partial + range[w];
-    staged[p] = partial;
-    __syncthreads();
-    if (p == 0) {
-      float s = -0.0f;
-      for (uint32_t q = 0; q < participants; ++q) s = s + staged[q];
-      total = total + s;
-    }
-    __syncthreads();
-  }
-  if (p == 0) out[blockIdx.x] = canon(total);
+  __shared__ __align__(16) float lds[kCoopFloats + 1024];  // the stage, then the partials
+  coop_rows<false>(x, gridDim.x, extent, participants, chunk, rounds, participant_major, out, false,
+                   [](float v) { return v; }, [](float acc, float t) { return acc + t; }, lds);
 }
-
-// The same under a FoldRule (evaluate.rs:845-1158 cooperative_grouped_sum_under):
-// every cell, the staged partials and the round totals seeded at their first
-// value.
 extern "C" __global__ void __launch_bounds__(1024)
 tiler_sum_f32_cooperative_m(const float* __restrict__ x, uint64_t extent, uint32_t participants,
                             uint64_t chunk, uint64_t rounds, uint32_t participant_major,
                             float* __restrict__ out, tiler::FoldRule rule) {
-  __shared__ float staged[1024];
-  const uint32_t p = threadIdx.x;
-  const float* row = x + (uint64_t)blockIdx.x * extent;
-  float total = 0.0f;
-  for (uint64_t r = 0; r < rounds; ++r) {
-    uint64_t cell = participant_major ? (uint64_t)p * rounds + r : r * participants + p;
-    const float* range = row + cell * chunk;
-    float partial = tiler::fold_contributor(rule, range[0]);
-    for (uint64_t w = 1; w < chunk; ++w) partial = tiler::fold_combine(rule, partial, tiler::fold_contributor(rule, range[w]));
-    staged[p] = partial;
-    __syncthreads();
-    if (p == 0) {
-      float s = staged[0];
-      for (uint32_t q = 1; q < participants; ++q) s = tiler::fold_combine(rule, s, staged[q]);
-      total = r == 0 ? s : tiler::fold_combine(rule, total, s);
-    }
-    __syncthreads();
-  }
-  if (p == 0) out[blockIdx.x] = canon(total);
+  __shared__ __align__(16) float lds[kCoopFloats + 1024];
+  coop_rule_rows<false>(x, gridDim.x, extent, participants, chunk, rounds, participant_major, out, rule, lds);
+}
+extern "C" __global__ void __launch_bounds__(256)
+tiler_sum_f32_cooperative_packed(const float* __restrict__ x, uint64_t rows, uint64_t extent, uint32_t participants,
+                                 uint64_t chunk, float* __restrict__ out) {
+  __shared__ __align__(16) float lds[kCoopFloats + 1024];
+  coop_rows<true>(x, rows, extent, participants, chunk, 1, 0, out, false, [](float v) { return v; },
+                  [](float acc, float t) { return acc + t; }, lds);
+}
+extern "C" __global__ void __launch_bounds__(256)
+tiler_sum_f32_cooperative_packed_m(const float* __restrict__ x, uint64_t rows, uint64_t extent,
+                                   uint32_t participants, uint64_t chunk, float* __restrict__ out,
+                                   tiler::FoldRule rule) {
+  __shared__ __align__(16) float lds[kCoopFloats + 1024];
+  coop_rule_rows<true>(x, rows, extent, participants, chunk, 1, 0, out, rule, lds);
 }
 
 // ---------------------------------------------------------------------------

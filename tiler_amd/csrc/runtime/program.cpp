@@ -200,6 +200,11 @@ static void add_serial_fold(const Target& t, uint32_t src, bool src_aligned, uin
       .ptr(src).u64(nrows).u64(length).u64(1).ptr(dst);
 }
 
+// Threads of a workgroup that packs rows of a one-round cooperative sum.  Eight
+// rows per CU and up, so that packing leaves every CU its workgroups; packed
+// against one row to a workgroup, us: 65536 rows of 16 participants 14.8 / 130,
+// 4096 of 64 19.0 / 25.8, 30000 of 20 21.6 / 144.
+constexpr uint32_t kCoopPackedThreads = 256;
 tiler_hip_status plan_sum_f32(const Target& t, uint64_t rows, uint64_t extent,
                               const tiler_hip_sum_plan& sp, const uintptr_t* addr, Program& p,
                               const FoldRuleHost* rule) {
@@ -247,6 +252,15 @@ tiler_hip_status plan_sum_f32(const Target& t, uint64_t rows, uint64_t extent,
       if (P == 0 || P > 1024 || c == 0 || R == 0 || P * c * R != extent)
         return p.refuse(TILER_HIP_REFUSE_INVALID_ARGUMENT, "grouping does not cover the axis exactly");
       if (rows > 0x7fffffffull) return p.refuse(TILER_HIP_REFUSE_CAPACITY, "more rows than the launch grid holds");
+      if (R == 1 && 2 * P <= kCoopPackedThreads && rows >= 8ull * t.compute_units) {
+        // many rows of small groups: whole rows packed into a workgroup
+        const uint32_t per = (uint32_t)(kCoopPackedThreads / P);
+        Launch& l = p.add(rule ? "tiler_sum_f32_cooperative_packed_m" : "tiler_sum_f32_cooperative_packed",
+                          (uint32_t)((rows + per - 1) / per), 1, (uint32_t)(per * P))
+                        .ptr(x).u64(rows).u64(extent).u32((uint32_t)P).u64(c).ptr(out);
+        if (rule) l.blob(rule, sizeof(*rule), 4);
+        return TILER_HIP_OK;
+      }
       Launch& l = p.add(rule ? "tiler_sum_f32_cooperative_m" : "tiler_sum_f32_cooperative", (uint32_t)rows, 1, (uint32_t)P)
                       .ptr(x).u64(extent).u32((uint32_t)P).u64(c).u64(R).u32(sp.participant_major ? 1u : 0u).ptr(out);
       if (rule) l.blob(rule, sizeof(*rule), 4);
