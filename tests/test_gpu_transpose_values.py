@@ -1,0 +1,54 @@
+"""The value contraction's right operand stored [k, n] (transposed ahead of the
+MFMA kernels): 16-byte and 2-byte forms of the transpose at the edges of its
+64 x 64 tiles, and its scratch across calls of growing and shrinking size.
+Operands are small integers, so the results are exact whatever the order."""
+import numpy as np
+import pytest
+
+import oracle
+from tiler_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ctx, m, k, n, batches=3, stream=None):
+    rng = np.random.default_rng(m + 3 * k + n)
+    p = rng.integers(-3, 4, (batches, m, k)).astype(np.float32)
+    v = rng.integers(-3, 4, (batches, k, n)).astype(np.float32)
+    want = np.matmul(p.astype(np.float64), v.astype(np.float64)).astype(np.float32)
+    s = L.contraction_structure("bmk", p.shape, "bkn", v.shape, "bmn")
+    bufs = [ctx.to_device(oracle.bf16_narrow(p)), ctx.to_device(oracle.bf16_narrow(v)), ctx.alloc(want.size * 2)]
+    try:
+        ctx.contract(L.BF16, s, *bufs, permissions=L.PERMITS_REASSOCIATION, stream=stream)
+        ctx.synchronize()
+        got = bufs[2].download(np.uint16, want.shape)
+    finally:
+        for b in bufs:
+            b.free()
+    assert np.array_equal(got, oracle.bf16_narrow(want).reshape(want.shape))
+
+
+@pytest.mark.parametrize("k,n", [(64, 64), (72, 40), (8, 8), (136, 128), (200, 72),  # 16 bytes a lane
+                                 (65, 64), (64, 41), (7, 3)])                        # 2 bytes
+def test_transposed_right_operand(ctx, k, n):
+    _check(ctx, 5, k, n)
+
+
+def test_scratch_across_sizes(ctx):
+    for k, n in ((64, 64), (1024, 520), (64, 72), (2048, 1032), (40, 8), (1024, 520)):
+        _check(ctx, 9, k, n, batches=2)
+
+
+def test_kept_widening_is_exact(ctx):
+    """Results of 32 MiB and up take the form with ordinary stores."""
+    n = (8 << 20) + 5
+    x = np.random.default_rng(3).integers(0, 1 << 16, n).astype(np.uint16)
+    dx, dy = ctx.to_device(x), ctx.alloc(4 * n)
+    try:
+        ctx.convert(L.CONVERT_WIDEN_BF16_F32, dx, n, dy)
+        ctx.synchronize()
+        got = dy.download(np.uint32, (n,))
+    finally:
+        dx.free()
+        dy.free()
+    assert np.array_equal(got, x.astype(np.uint32) << 16)

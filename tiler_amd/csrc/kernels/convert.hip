@@ -46,8 +46,8 @@ tiler_narrow_f32_bf16(const float* __restrict__ x, uint64_t n, uint16_t* __restr
 }
 
 // n8 groups of 8 elements: one 16-byte bf16 chunk in, two f32x4 out.
-extern "C" __global__ void __launch_bounds__(256)
-tiler_widen_bf16_f32_v8(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
+template <bool kKeep>
+__device__ __forceinline__ void widen_v8(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += stride) {
     const u32x4 v = __builtin_nontemporal_load(&x[i]);
@@ -55,9 +55,22 @@ tiler_widen_bf16_f32_v8(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restr
                      __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
     const f32x4 b = {__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xffff0000u),
                      __uint_as_float(v.w << 16), __uint_as_float(v.w & 0xffff0000u)};
-    __builtin_nontemporal_store(a, &y[2 * i]);
-    __builtin_nontemporal_store(b, &y[2 * i + 1]);
+    tiler::store_result<kKeep>(a, &y[2 * i]);
+    tiler::store_result<kKeep>(b, &y[2 * i + 1]);
   }
+}
+
+extern "C" __global__ void __launch_bounds__(256)
+tiler_widen_bf16_f32_v8(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
+  widen_v8<false>(x, n8, y);
+}
+// The same with ordinary stores, for results of 32 MiB and up: the pass that
+// reads them next finds what the caches hold, and the widening itself is no
+// slower (2^26 elements 82 against 90 us; 2^22, 16 MiB, 7.4 against 6.2, which
+// is why smaller ones stream).
+extern "C" __global__ void __launch_bounds__(256)
+tiler_widen_bf16_f32_v8_c(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
+  widen_v8<true>(x, n8, y);
 }
 
 extern "C" __global__ void __launch_bounds__(256)

@@ -147,11 +147,12 @@ tiler_map_bf16(const uint16_t* __restrict__ x, const uint16_t* __restrict__ x2,
 }
 
 // Vectorized maps: 16 bytes per lane per step (4 f32 or 8 bf16 elements),
-// non-temporal loads and stores, the op and the rank-0 broadcast of x2 fixed at
-// compile time.  Every element sees exactly the scalar kernels' arithmetic.
+// non-temporal loads and stores (f32 results of 32 to 128 MiB: ordinary stores,
+// tiler::keep_in_cache), the op and the rank-0 broadcast of x2 fixed at compile
+// time.  Every element sees exactly the scalar kernels' arithmetic.
 // The host uses them on 16-byte-aligned operands for the whole 16-byte chunks
 // and the scalar kernels for the tail.
-template <uint32_t OP, bool BCAST>
+template <uint32_t OP, bool BCAST, bool kKeep>
 __device__ __forceinline__ void map_f32_v4_body(const f32x4* __restrict__ x, const float* __restrict__ x2,
                                                 uint64_t n4, float a, float b, f32x4* __restrict__ y) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -162,7 +163,7 @@ __device__ __forceinline__ void map_f32_v4_body(const f32x4* __restrict__ x, con
     if (OP >= 2 && !BCAST) s2 = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(x2) + i);
     const f32x4 o = {map_op(OP, v.x, s2.x, a, b), map_op(OP, v.y, s2.y, a, b),
                      map_op(OP, v.z, s2.z, a, b), map_op(OP, v.w, s2.w, a, b)};
-    __builtin_nontemporal_store(o, &y[i]);
+    tiler::store_result<kKeep>(o, &y[i]);
   }
 }
 
@@ -192,7 +193,8 @@ __device__ __forceinline__ void map_bf16_v8_body(const u32x4* __restrict__ x, co
   extern "C" __global__ void __launch_bounds__(256) tiler_map_f32_v4_op##OP##SFX(                    \
       const f32x4* __restrict__ x, const float* __restrict__ x2, uint64_t n4, float a, float b,      \
       f32x4* __restrict__ y) {                                                                       \
-    map_f32_v4_body<OP, BC>(x, x2, n4, a, b, y);                                                     \
+    if (tiler::keep_in_cache(n4 * 16u)) map_f32_v4_body<OP, BC, true>(x, x2, n4, a, b, y);            \
+    else map_f32_v4_body<OP, BC, false>(x, x2, n4, a, b, y);                                         \
   }                                                                                                  \
   extern "C" __global__ void __launch_bounds__(256) tiler_map_bf16_v8_op##OP##SFX(                   \
       const u32x4* __restrict__ x, const uint16_t* __restrict__ x2, uint64_t n8, float a, float b,   \

@@ -193,6 +193,7 @@ const EntryRow kEntries[] = {
     {"tiler_narrow_f32_bf16_v8", "convert-f32-to-bf16/narrow", 2},
     {"tiler_narrow_f32_bf16", "convert-f32-to-bf16/narrow", 2},
     {"tiler_widen_bf16_f32_v8", "convert-bf16-to-f32/widen", 2},
+    {"tiler_widen_bf16_f32_v8_c", "convert-bf16-to-f32/widen", 2},
     {"tiler_widen_bf16_f32", "convert-bf16-to-f32/widen", 2},
     {"tiler_dequantize_u4_f32_w", "dequantize-strict-affine-u4", 2},
     {"tiler_dequantize_u4_f32_v4", "dequantize-strict-affine-u4", 2},
