@@ -39,6 +39,45 @@ def test_scratch_across_sizes(ctx):
         _check(ctx, 9, k, n, batches=2)
 
 
+def test_scratch_of_other_streams_and_threads(ctx):
+    """Calls on another stream take scratch of their own; calls from two
+    threads on the context's stream do not interleave over the kept one."""
+    import threading
+
+    import tiler_amd
+    with tiler_amd.Context(0) as other:
+        for _ in range(4):
+            _check(ctx, 33, 520, 136)  # the context's stream
+            rng = np.random.default_rng(5)
+            p = rng.integers(-3, 4, (2, 7, 72)).astype(np.float32)
+            v = rng.integers(-3, 4, (2, 72, 40)).astype(np.float32)
+            want = np.matmul(p, v)
+            s = L.contraction_structure("bmk", p.shape, "bkn", v.shape, "bmn")
+            bufs = [ctx.to_device(oracle.bf16_narrow(p)), ctx.to_device(oracle.bf16_narrow(v)),
+                    ctx.alloc(want.size * 2)]
+            ctx.contract(L.BF16, s, *bufs, permissions=L.PERMITS_REASSOCIATION, stream=other.stream)
+            other.synchronize()
+            got = bufs[2].download(np.uint16, want.shape)
+            for b in bufs:
+                b.free()
+            assert np.array_equal(got, oracle.bf16_narrow(want).reshape(want.shape))
+    errors = []
+
+    def work(k, n):
+        try:
+            for _ in range(8):
+                _check(ctx, 17, k, n)
+        except BaseException as e:  # noqa: BLE001 (reported by the main thread)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=a) for a in ((520, 264), (72, 1032))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
 def test_kept_widening_is_exact(ctx):
     """Results of 32 MiB and up take the form with ordinary stores."""
     n = (8 << 20) + 5

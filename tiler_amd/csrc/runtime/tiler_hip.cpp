@@ -4,6 +4,7 @@
 // hipModuleLoadData and every launch goes through hipModuleLaunchKernel.
 #include "tiler_hip.h"
 
+#include <mutex>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -387,6 +388,12 @@ struct tiler_hip_context {
   // workspace: [partials kWorkspacePartialBytes][gather_bad u64 + pad]
   //            [row-synchronized softmax area kRowSyncBytes: epoch, tagged words]
   uint8_t* workspace = nullptr;
+  // Scratch of the direct calls that need more than the workspace holds, kept
+  // between calls on the context's own stream (which orders its users): see
+  // CallScratch.
+  std::mutex scratch_mutex;
+  void* scratch = nullptr;
+  uint64_t scratch_bytes = 0;
   float* sum_partials = nullptr;
   unsigned long long* gather_bad = nullptr;
   uint8_t* row_sync = nullptr;
@@ -470,6 +477,49 @@ bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
+
+// Scratch for one direct call.  On the context's own stream, up to
+// kScratchKept bytes come from a buffer the context keeps: allocating and
+// freeing it on the stream for every call cost more than the kernels of a
+// small one (the pool gives memory back at each synchronization, so a call
+// that is waited for pays the allocation again).  The buffer grows in powers
+// of two, the outgrown one freed in stream order behind the calls that use it.
+// The lock is held until the call has enqueued everything, so that calls from
+// two threads cannot interleave their launches over the one buffer.  Other
+// streams and larger requests allocate on the stream for the call alone.
+constexpr uint64_t kScratchKept = 64ull << 20;
+class CallScratch {
+ public:
+  CallScratch(tiler_hip_context* ctx, hipStream_t s) : ctx_(ctx), s_(s) {}
+  ~CallScratch() {
+    if (own_) hipFreeAsync(own_, s_);
+  }
+  CallScratch(const CallScratch&) = delete;
+  CallScratch& operator=(const CallScratch&) = delete;
+  void* get(uint64_t bytes) {  // null when the allocation fails
+    if (s_ != ctx_->stream || bytes > kScratchKept) {
+      if (hipMallocAsync(&own_, bytes, s_) != hipSuccess) own_ = nullptr;
+      return own_;
+    }
+    lock_ = std::unique_lock<std::mutex>(ctx_->scratch_mutex);
+    if (ctx_->scratch_bytes < bytes) {
+      uint64_t grown = 1ull << 20;
+      while (grown < bytes) grown <<= 1;
+      void* fresh = nullptr;
+      if (hipMallocAsync(&fresh, grown, s_) != hipSuccess) return nullptr;
+      if (ctx_->scratch) hipFreeAsync(ctx_->scratch, s_);
+      ctx_->scratch = fresh;
+      ctx_->scratch_bytes = grown;
+    }
+    return ctx_->scratch;
+  }
+
+ private:
+  tiler_hip_context* ctx_;
+  hipStream_t s_;
+  void* own_ = nullptr;
+  std::unique_lock<std::mutex> lock_;
+};
 
 tiler_rt::Target target_of(const tiler_hip_context* ctx) {
   return tiler_rt::Target{ctx ? ctx->compute_units : kProfileComputeUnits,
@@ -971,6 +1021,7 @@ void tiler_hip_release(tiler_hip_context* ctx) {
   for (auto& kv : ctx->expression_programs) hipFree(kv.second);
   if (ctx->module) hipModuleUnload(ctx->module);
   if (ctx->workspace) hipFree(ctx->workspace);
+  if (ctx->scratch) hipFree(ctx->scratch);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -1478,8 +1529,8 @@ tiler_hip_status tiler_hip_sum_f32(tiler_hip_context* ctx, const float* x, uint6
   hipStream_t s = pick(ctx, stream);
   void* slots[tiler_rt::kMaxSlots] = {const_cast<float*>(x), out, nullptr};
   // Partials live in the context workspace when they fit (ordered on the
-  // stream); only larger splits allocate, stream-ordered.
-  bool own = false;
+  // stream); larger splits take call scratch.
+  CallScratch scratch(ctx, s);
   if (p.nslots > 2 && p.nlaunches) {
     if (p.slot_bytes[2] <= tiler_rt::kWorkspacePartialBytes) {
       if ((st = workspace_stream(ctx, stream, "this sum's partials")) != TILER_HIP_OK) return st;
@@ -1487,14 +1538,11 @@ tiler_hip_status tiler_hip_sum_f32(tiler_hip_context* ctx, const float* x, uint6
     } else {
       if (capturing(s))
         return fail(ctx, TILER_HIP_REFUSE_CAPACITY, "partials exceed the workspace under graph capture");
-      if (hipMallocAsync(&slots[2], p.slot_bytes[2], s) != hipSuccess)
+      if (!(slots[2] = scratch.get(p.slot_bytes[2])))
         return fail(ctx, TILER_HIP_FAIL_ALLOCATION, "partials allocation failed");
-      own = true;
     }
   }
-  st = run_program(ctx, p, slots, s);
-  if (own) hipFreeAsync(slots[2], s);
-  return st;
+  return run_program(ctx, p, slots, s);
 } catch (...) {  // host memory exhausted: nothing unwinds through the C ABI
   return TILER_HIP_REFUSE_CAPACITY;
 }
@@ -1554,9 +1602,9 @@ tiler_hip_status tiler_hip_softmax_f32(tiler_hip_context* ctx, const float* x, u
   hipStream_t s = pick(ctx, stream);
   void* slots[tiler_rt::kMaxSlots] = {const_cast<float*>(x), y};
   // The split form's partials (segment maxima, then sums) live in the context
-  // workspace when they fit (ordered on the stream); larger ones are
-  // allocated, stream-ordered.
-  bool own = false;
+  // workspace when they fit (ordered on the stream); larger ones take call
+  // scratch.
+  CallScratch scratch(ctx, s);
   uint8_t* part = nullptr;
   if (p.nslots == 3) {  // the row-synchronized form: its area in the workspace
     if (p.slot_bytes[2] > tiler_rt::kRowSyncBytes) return fail(ctx, TILER_HIP_REFUSE_CAPACITY, "row-sync area");
@@ -1570,16 +1618,13 @@ tiler_hip_status tiler_hip_softmax_f32(tiler_hip_context* ctx, const float* x, u
     } else {
       if (capturing(s))
         return fail(ctx, TILER_HIP_REFUSE_CAPACITY, "partials exceed the workspace under graph capture");
-      if (hipMallocAsync(reinterpret_cast<void**>(&part), bytes, s) != hipSuccess)
+      if (!(part = static_cast<uint8_t*>(scratch.get(bytes))))
         return fail(ctx, TILER_HIP_FAIL_ALLOCATION, "partials allocation failed");
-      own = true;
     }
     slots[2] = part;
     slots[3] = part + p.slot_bytes[2];
   }
-  st = run_program(ctx, p, slots, s);
-  if (own) hipFreeAsync(part, s);
-  return st;
+  return run_program(ctx, p, slots, s);
 } catch (...) {  // host memory exhausted: nothing unwinds through the C ABI
   return TILER_HIP_REFUSE_CAPACITY;
 }
@@ -1770,21 +1815,18 @@ tiler_hip_status tiler_hip_contract(tiler_hip_context* ctx, uint32_t dtype,
   if (!left || !right || !out) return TILER_HIP_REFUSE_INVALID_ARGUMENT;
   hipStream_t s = pick(ctx, stream);
   void* slots[tiler_rt::kMaxSlots] = {const_cast<void*>(left), const_cast<void*>(right), out};
-  bool own = false;
+  CallScratch scratch(ctx, s);
   if (p.nslots > 3) {
     if (p.slot_roles[3] == TILER_HIP_SLOT_CONSTANT) {
       st = resident_constant(ctx, p, s, &slots[3]);
       if (st != TILER_HIP_OK) return st;
     } else {  // the transposed right operand
       if (capturing(s)) return fail(ctx, TILER_HIP_REFUSE_CAPACITY, "transpose workspace allocation under graph capture");
-      if (hipMallocAsync(&slots[3], p.slot_bytes[3], s) != hipSuccess)
+      if (!(slots[3] = scratch.get(p.slot_bytes[3])))
         return fail(ctx, TILER_HIP_FAIL_ALLOCATION, "transpose workspace allocation failed");
-      own = true;
     }
   }
-  st = run_program(ctx, p, slots, s);
-  if (own) hipFreeAsync(slots[3], s);
-  return st;
+  return run_program(ctx, p, slots, s);
 } catch (...) {  // host memory exhausted: nothing unwinds through the C ABI
   return TILER_HIP_REFUSE_CAPACITY;
 }
@@ -1820,16 +1862,13 @@ tiler_hip_status tiler_hip_expression(tiler_hip_context* ctx, uint32_t dtype,
   if (st != TILER_HIP_OK) return st;
   for (uint32_t k = 0; k < prog.inputs; ++k) slots[k] = const_cast<void*>(inputs[k]);
   slots[prog.inputs] = y;
-  bool own = false;
+  CallScratch scratch(ctx, s);
   if (p.nslots > prog.inputs + 2) {  // the value store
     if (capturing(s)) return fail(ctx, TILER_HIP_REFUSE_CAPACITY, "value store allocation under graph capture");
-    if (hipMallocAsync(&slots[prog.inputs + 2], p.slot_bytes[prog.inputs + 2], s) != hipSuccess)
+    if (!(slots[prog.inputs + 2] = scratch.get(p.slot_bytes[prog.inputs + 2])))
       return fail(ctx, TILER_HIP_FAIL_ALLOCATION, "value store allocation failed");
-    own = true;
   }
-  st = run_program(ctx, p, slots, s);
-  if (own) hipFreeAsync(slots[prog.inputs + 2], s);
-  return st;
+  return run_program(ctx, p, slots, s);
 } catch (...) {  // host memory exhausted: nothing unwinds through the C ABI
   return TILER_HIP_REFUSE_CAPACITY;
 }
