@@ -1,4 +1,4 @@
-"""The strict f32 contraction's column-per-lane forms (4 and 16 rows to 64
+"""The strict f32 contraction's column-per-lane forms (1, 4 and 16 rows to 64
 columns) and the 64 x 64 tiles, at the edges of their tiles and of the 64-step
 stages of k, bit for bit with the oracle's first-product fold
 (tiler-reference/src/contraction.rs:558-630)."""
@@ -11,6 +11,7 @@ from tiler_amd.realize import realize
 
 CASES = [
     (17, 63, 64, "b16"), (18, 65, 65, "b16"), (20, 64, 128, "b16"), (33, 130, 191, "b16"), (19, 7, 260, "b16"),
+    (10, 2049, 128, "s64"), (16, 1000, 191, "s64"), (2, 8191, 66, "s64"), (9, 1100, 1024, "s64"),
     (250, 1030, 100, "b32"), (273, 1000, 131, "b32"), (289, 2049, 64, "b32"), (2048, 2047, 66, "b64"),
 ]
 
@@ -23,6 +24,7 @@ def test_form_choice(m, n, k, form):
 
 def test_long_k_keeps_64_bit_addresses():
     assert realize(L.PROGRAM_CONTRACTION, (17, 2, 1 << 24)).symbols == ["tiler_contract_strict_f32_b64"]
+    assert realize(L.PROGRAM_CONTRACTION, (16, 1 << 20, 1 << 24)).symbols == ["tiler_contract_strict_f32_s16"]
 
 
 @pytest.mark.gpu
@@ -33,8 +35,8 @@ def test_columns_match_the_strict_fold(ctx, m, n, k, form):
     b = rng.standard_normal((n, k)).astype(np.float32)
     a[m - 1] = -0.0                      # products of zeros keep their sign through the seed
     b[0] = np.abs(b[0])
-    a[2, k - 1], b[n - 1, 0] = np.inf, np.nan
-    a[5] *= np.float32(1e-30)
+    a[0, k - 1], b[n - 1, 0] = np.inf, np.nan
+    a[m // 2] *= np.float32(1e-30)
     b[n // 2] *= np.float32(1e-12)       # subnormal products
     want = oracle.contract_strict_f32(a, b, m, n, k).reshape(m, n)
     dc = ctx.alloc(4 * m * n + 64)

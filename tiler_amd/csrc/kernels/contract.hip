@@ -181,14 +181,15 @@ __device__ __forceinline__ void contract_strict_blocked_body(const T* __restrict
 // before the current ones are folded (the s_waitcnt at the head of a block
 // covers both kinds, which share a counter and return in any order).  The same
 // ascending first-product fold; steps past k are never folded, rows past m
-// read the last one and are not stored.
+// read the last one and are not stored.  FW < W: only the first FW waves fold
+// (TM FW rows), the others load.
 //
 // Bound by VALU issue where the chip is full (512 x 3072 x 1024: 70 us, 46 T
 // operations/s; the register-blocked 32 x 32 tiles took 113), else by the
 // latency of a block's operands.  Before and now, us: 17 x 1024 x 1024
 // 29 / 10.2, 128 x 3072 x 1024 49 / 27, 128 x 1024 x 3072 90 / 34,
 // 256 x 1024 x 1024 44 / 17.6, 300 x 3000 x 2000 285 / 111.
-template <int TM, int KB, int W>
+template <int TM, int KB, int W, int FW = W>
 __device__ __forceinline__ void contract_strict_columns_body(const float* __restrict__ a,
                                                              const float* __restrict__ b, uint32_t m, uint32_t n,
                                                              uint32_t k, float* __restrict__ c, uint32_t row0,
@@ -245,37 +246,40 @@ __device__ __forceinline__ void contract_strict_columns_body(const float* __rest
   for (int i = 0; i < TM; ++i) acc[i] = -0.0f;  // -0 + first product == first product
   const uint32_t stages = (k + 63u) / 64u, whole = k / 64u;
   issue(0);
-  if (whole) load_a(av[0], 0);
+  const bool folds = FW == W || wave < (uint32_t)FW;
+  if (whole && folds) load_a(av[0], 0);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   for (uint32_t s = 0; s < whole; ++s) {
     if (s + 1 < stages) issue(s + 1);  // into the buffer every wave left at the last barrier
     const float* src = stage + (s & 1u) * 4096u + lane * 64u;
-    load_b(bv[0], src, 0);
-    const uint32_t next = s + 1 < whole ? (s + 1) * 64u : 0u;
-    auto block = [&](auto kbs) -> bool {
-      constexpr int kb = decltype(kbs)::value, p = kb & 1;
-      __builtin_amdgcn_s_waitcnt(kLgkm0);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kb + 1 < kBlk) {
-        load_a(av[p ^ 1], s * 64u + (kb + 1) * KB);
-        load_b(bv[p ^ 1], src, kb + 1);
-      } else {
-        load_a(av[p ^ 1], next);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+    if (folds) {
+      load_b(bv[0], src, 0);
+      const uint32_t next = s + 1 < whole ? (s + 1) * 64u : 0u;
+      auto block = [&](auto kbs) -> bool {
+        constexpr int kb = decltype(kbs)::value, p = kb & 1;
+        __builtin_amdgcn_s_waitcnt(kLgkm0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kb + 1 < kBlk) {
+          load_a(av[p ^ 1], s * 64u + (kb + 1) * KB);
+          load_b(bv[p ^ 1], src, kb + 1);
+        } else {
+          load_a(av[p ^ 1], next);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int e = 0; e < KB; ++e)
+        for (int e = 0; e < KB; ++e)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) acc[i] = acc[i] + av[p][i][e] * bv[p][e / 4][e % 4];
-      __builtin_amdgcn_sched_barrier(0);
-      return true;
-    };
-    tiler::unrolled_while<0, kBlk>(block);
+          for (int i = 0; i < TM; ++i) acc[i] = acc[i] + av[p][i][e] * bv[p][e / 4][e % 4];
+        __builtin_amdgcn_sched_barrier(0);
+        return true;
+      };
+      tiler::unrolled_while<0, kBlk>(block);
+    }
     // this wave's share of stage s + 1 has landed; its reads of stage s were
     // waited for at the head of the last block
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   }
-  if (whole < stages) {
+  if (whole < stages && folds) {
     const float* src = stage + (whole & 1u) * 4096u + lane * 64u;
     const uint32_t count = k - whole * 64u;
     for (uint32_t e = 0; e < count; ++e) {
@@ -284,7 +288,7 @@ __device__ __forceinline__ void contract_strict_columns_body(const float* __rest
       for (int i = 0; i < TM; ++i) acc[i] = acc[i] + ar[i][whole * 64u + e] * bw;
     }
   }
-  if (lane < cols) {
+  if (lane < cols && folds) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const uint32_t r = row0 + wave * TM + i;
@@ -337,8 +341,11 @@ tiler_contract_strict_f32_b64(const float* __restrict__ a, const float* __restri
 // (tiler_sum_f32_staged_r*, reduce.hip) of the products of A's row i with B's
 // rows, which are contiguous in k -- the same first-product fold, ascending k,
 // two roundings per step, bit for bit.  R output columns per workgroup; R in
-// {1, 4, 16} relay-fold the staged products (staged_relay_body), R = 64 folds
-// a row per lane (staged_fold_body).
+// {1, 4, 16} relay-fold the staged products (staged_relay_body), R = 64 is the
+// column-per-lane form with one folding wave of the four, at any alignment (a
+// row's product per lane, both operands through LDS, took 15.7 us at
+// 10 x 2048 x 1024 and 41.4 at 16 x 1024 x 3072; 9.7 and 30.0 now;
+// 1 x 151936 x 1024 134 -> 128).
 #define TILER_CONTRACT_STRICT_ROWS(R, BODY)                                                            \
   extern "C" __global__ void __launch_bounds__(256)                                                    \
       tiler_contract_strict_f32_s##R(const float* __restrict__ a, const float* __restrict__ b,          \
@@ -357,7 +364,11 @@ tiler_contract_strict_f32_b64(const float* __restrict__ a, const float* __restri
 TILER_CONTRACT_STRICT_ROWS(1, staged_relay_body)
 TILER_CONTRACT_STRICT_ROWS(4, staged_relay_body)
 TILER_CONTRACT_STRICT_ROWS(16, staged_relay_body)
-TILER_CONTRACT_STRICT_ROWS(64, staged_lane_body)
+extern "C" __global__ void __launch_bounds__(256)
+tiler_contract_strict_f32_s64(const float* __restrict__ a, const float* __restrict__ b, uint32_t m, uint32_t n,
+                              uint32_t k, float* __restrict__ c) {
+  contract_strict_columns_body<1, 32, 4, 1>(a, b, m, n, k, c, blockIdx.y, blockIdx.x * 64u);
+}
 
 // ---------------------------------------------------------------------------
 // bf16 MFMA contraction.

@@ -213,7 +213,6 @@ const EntryRow kEntries[] = {
     {"tiler_contract_strict_f32_s16", "tensor-contraction-f32/strict", 3},
     {"tiler_contract_strict_f32_s16_u", "tensor-contraction-f32/strict", 3},
     {"tiler_contract_strict_f32_s64", "tensor-contraction-f32/strict", 3},
-    {"tiler_contract_strict_f32_s64_u", "tensor-contraction-f32/strict", 3},
     {"tiler_contract_strict_bf16", "tensor-contraction-bf16/strict", 3},
     {"tiler_contract_strict_bf16_silu", "tensor-contraction-bf16/strict+silu", 3},
     {"tiler_contract_strict_bf16_b16", "tensor-contraction-bf16/strict", 3},
