@@ -842,36 +842,39 @@ static uint64_t ksplit_grid(uint64_t m, uint64_t n, uint32_t mb, uint32_t nb) {
 }
 
 // The k-split tile for `batches` products of m x n x k, or null where the
-// 128- or 256-tiles are the better form.  Times in ns, fitted on the device
-// over m 65..3000 and n, k 616..8192 (root mean square error 14%; the choice
-// costs 1% over the best of the tiles and the staged forms):
+// 128- or 256-tiles are the better form.  Only where the 128-tiles do not go
+// round the CUs once: beyond, several rounds of tiles share the L2s badly
+// (3000 x 4096 x 4096 146 us in 6 x 8 tiles against 115, 3000 x 2049 x 1024 55
+// in 5 x 4 against 28 in the general form).  Within, times in ns, fitted on the
+// device over m 65..3000 and n, k 616..8192 (the choice costs 0.6% over the
+// best of the tiles and the staged forms, and none is slower than the latter):
 // * k-split: 2400 + rounds of tiles over the CUs x (0.392 k (MB + NB), the
-//   operand fill, + 136 per block, the fold of the partial tiles); two
+//   operand fill, a fifth more where the 64-deep chunks straddle 128-byte
+//   lines, + 136 per block, the fold of the partial tiles).  The rounds are
+//   those of the XCD with the most panels (1045 x 2536 x 2248 in 6 x 8 tiles:
+//   220 tiles, 33 on some XCDs of 32 CUs, 47 us against 34 staged); two
 //   workgroups of at most 80 KiB share a CU, so a part round costs them less;
-// * 128-tiles: 3400 + 660 per 64-deep k tile, 1050 with two tiles on a CU;
-//   twice that in the general form, which serves n off the 8-element grid.
+// * 128-tiles: 3400 + 660 per 64-deep k tile, twice that in the general form,
+//   which serves n off the 8-element grid.
 // A k-split tile has to be a tenth faster by these to be taken.  From k = 512
 // on each of eight waves has a chunk of its own.
 static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batches) {
   if (k < 512 || k >= (1ull << 24)) return nullptr;
   const uint64_t cus = t.compute_units;
-  const uint64_t t256 = mul_sat(mul_sat((m + 255) / 256, (n + 255) / 256), batches);
-  if (t256 >= cus) return nullptr;
   const uint64_t t128 = mul_sat(mul_sat((m + 127) / 128, (n + 127) / 128), batches);
-  const uint64_t steps = (k + 63) / 64;
-  uint64_t staged = 3400 + (t128 <= cus ? 660 * steps : 1050 * steps * ((t128 + 2 * cus - 1) / (2 * cus)));
-  if (n % 8 != 0) staged *= 2;
+  if (t128 > cus) return nullptr;
+  const uint64_t staged = (3400 + 660 * ((k + 63) / 64)) * (n % 8 != 0 ? 2 : 1);
   const KsplitTile* best = nullptr;
   uint64_t best_ns = staged * 9 / 10;
   for (const KsplitTile& c : kKsplitTiles) {
-    const uint64_t tm = (m + 16 * c.mb - 1) / (16 * c.mb), tn = (n + 16 * c.nb - 1) / (16 * c.nb);
-    const uint64_t tiles = tm * tn * batches;  // t256 < cus bounds all three
-    uint64_t rounds = (tiles + cus - 1) / cus * 1000;  // in thousandths
+    const uint64_t tiles = ksplit_grid(m, n, c.mb, c.nb) * batches;  // whole panel groups
+    uint64_t rounds = (tiles + cus - 1) / cus * 1000;                // in thousandths
     if ((c.mb + c.nb) * c.waves <= 40) {
       rounds = (660 * rounds + 340 * (tiles * 1000 / cus)) / 1000;
       if (rounds < 1000) rounds = 1000;
     }
-    const uint64_t ns = 2400 + rounds * (392 * k * (c.mb + c.nb) / 1000 + 136 * c.mb * c.nb) / 1000;
+    const uint64_t fill = (k % 64 != 0 ? 470 : 392) * k * (c.mb + c.nb) / 1000;
+    const uint64_t ns = 2400 + rounds * (fill + 136 * c.mb * c.nb) / 1000;
     if (ns < best_ns) best_ns = ns, best = &c;
   }
   return best;
