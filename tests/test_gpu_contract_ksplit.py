@@ -34,7 +34,7 @@ def test_staged_tiles_keep_the_large_products():
     for shape in ((4096, 4096, 4096), (2048, 4096, 4096), (1000, 2048, 512), (3000, 8192, 1024),
                   (3000, 4096, 4096), (1536, 3000, 3400), (1045, 2536, 2248)):
         rz = realize(L.PROGRAM_CONTRACTION, shape, dtype=L.BF16, permissions=RE)
-        assert rz.symbols[0] in ("tiler_contract_bf16_t256_kf", "tiler_contract_bf16_t128_kf"), shape
+        assert rz.symbols[0].startswith(("tiler_contract_bf16_t256", "tiler_contract_bf16_t128")), shape
     rz = realize(L.PROGRAM_CONTRACTION, (3000, 2049, 1024), dtype=L.BF16, permissions=RE)
     assert rz.symbols == ["tiler_contract_bf16_g128"]
 
