@@ -27,6 +27,12 @@ def test_long_k_keeps_64_bit_addresses():
     assert realize(L.PROGRAM_CONTRACTION, (16, 1 << 20, 1 << 24)).symbols == ["tiler_contract_strict_f32_s16"]
 
 
+def test_wide_n_stays_within_the_grid():
+    """2^32 work items along n do not fit a launch; a 64 x 64 tile per 256 threads does."""
+    assert realize(L.PROGRAM_CONTRACTION, (17, (1 << 28) - 64, 64)).symbols == ["tiler_contract_strict_f32_b32"]
+    assert realize(L.PROGRAM_CONTRACTION, (17, 1 << 28, 64)).symbols == ["tiler_contract_strict_f32_b64"]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,form", CASES)
 def test_columns_match_the_strict_fold(ctx, m, n, k, form):

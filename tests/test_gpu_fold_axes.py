@@ -41,6 +41,27 @@ def test_adjacent_axes_are_recognized(shape, mask, symbol):
     assert rz.symbols == [symbol]
 
 
+@pytest.mark.parametrize("shape,mask,variant,symbol", [
+    # 2^32 work items and more do not fit a launch: the grid-stride form takes them
+    ((1 << 28, 16), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    (((1 << 28) - 16, 16), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((1 << 26, 257), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    (((1 << 26) - 4, 257), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((1 << 24, 2048), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    (((1 << 24) - 2, 2048), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((1 << 30, 64), 0b10, L.FOLD_SUM, "tiler_fold_sum_f32"),
+    (((1 << 30) - 64, 64), 0b10, L.FOLD_SUM, "tiler_sum_f32_staged_r64"),
+    ((1 << 30, 64), 0b10, L.FOLD_SQUARED, "tiler_fold_squared_f32"),
+    ((1 << 30, 16), 0b10, L.FOLD_SUM, "tiler_sum_f32_staged_r256"),
+    ((1 << 16, 16, 1 << 16), 0b010, L.FOLD_SUM, "tiler_fold_sum_f32"),
+    ((1 << 16, 16, (1 << 16) - 1), 0b010, L.FOLD_SUM, "tiler_fold_sum_f32_lanes"),
+])
+def test_launches_stay_within_the_grid(shape, mask, variant, symbol):
+    rz = realize(L.PROGRAM_FOLD, shape, rank=len(shape), grouping=(mask,), variant=variant, flags=L.REGION_ALIGNED16)
+    assert rz.symbols == [symbol]
+    assert all(d.grid[0] * d.block[0] < 1 << 32 for d in rz.dispatches)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", COLS + LANES + ROWS)
 @pytest.mark.parametrize("variant", [L.FOLD_SUM, L.FOLD_SQUARED, L.FOLD_FMA, L.FOLD_MAXIMUM])

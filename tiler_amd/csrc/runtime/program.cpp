@@ -42,6 +42,10 @@ uint32_t blocks_capped(uint64_t work, uint64_t cap) {
   return (uint32_t)(b < cap ? b : cap);
 }
 
+// Whether one launch holds this many workgroups along x: the runtime takes
+// fewer than 2^32 work items.
+bool grid_holds(uint64_t workgroups, uint32_t threads) { return workgroups <= 0xffffffffull / threads; }
+
 // Host mirror of the kernels' BroadcastGeometry argument.
 struct BroadcastGeometryHost {
   uint64_t out_dims[8];
@@ -765,7 +769,7 @@ static uint32_t strict_tile(const Target& t, uint64_t m, uint64_t n) {
 enum class StrictForm { kRows4, kRows16, kTile64 };
 static StrictForm strict_f32_form(const Target& t, uint64_t m, uint64_t n, uint64_t k) {
   const uint64_t cus = t.compute_units, tn = (n + 63) / 64;
-  if (k >= (1ull << 24)) return StrictForm::kTile64;
+  if (k >= (1ull << 24) || !grid_holds(2 * tn, 512)) return StrictForm::kTile64;
   if (mul_sat(tn, (m + 3) / 4) <= 4 * cus) return StrictForm::kRows4;
   const uint64_t r16 = (mul_sat(tn, (m + 15) / 16) + cus - 1) / cus;
   const uint64_t r64 = (mul_sat(tn, (m + 63) / 64) + cus - 1) / cus;
@@ -1531,7 +1535,13 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
     // The reduced axes are adjacent: [outer, contributors, inner].
     char name[48];
     const uint64_t cus = t->compute_units;
-    if (inner == 1 && outputs <= 0x7fffffffull) {
+    // The maximum's lanes to a row: 16, a wave, or a workgroup for long or few
+    // rows.  The sums' staged forms take 64 rows to a workgroup, 256 of fewer
+    // than 64 elements (fewer where the rows are few).  More workgroups than a
+    // launch holds: the grid-stride form below.
+    const uint32_t lanes = contributors >= 2048 || outputs <= 4 * cus ? 256 : contributors > 256 ? 64 : 16;
+    const uint32_t per = op == TILER_HIP_FOLD_MAXIMUM ? 256 / lanes : contributors < 64 ? 256 : 64;
+    if (inner == 1 && grid_holds((outputs + per - 1) / per, 256)) {
       // contiguous rows: the staged strict sums (a prologue as a rule under
       // the preserving modes), or the maximum's row kernel
       if (op == TILER_HIP_FOLD_SUM) {
@@ -1546,9 +1556,6 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
         add_rule_fold(*t, x, aligned16(addr[x]), outputs, contributors, out, rule, p);
         return TILER_HIP_OK;
       }
-      // 16 lanes to a row, a wave, or a workgroup for long or few rows
-      const uint32_t lanes = contributors >= 2048 || outputs <= 4 * cus ? 256 : contributors > 256 ? 64 : 16;
-      const uint32_t per = 256 / lanes;
       p.add("tiler_fold_maximum_f32_rows", (uint32_t)((outputs + per - 1) / per), 1, 256)
           .ptr(x).ptr(out).u64(outputs).u64(contributors).u32(lanes);
       return TILER_HIP_OK;
@@ -1561,7 +1568,7 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
     // 81 / 11.8), and short folds do not fill a stage (300 x 50 x 1000
     // 97 / 11.7).  The columns' 32-bit offsets take inner below 2^21.
     const bool cols = contributors >= 128 && outputs <= 64 * cus && inner < (1ull << 21);
-    if (inner > 1 && (cols ? groups : blocks) <= 0x7fffffffull) {
+    if (inner > 1 && (cols || grid_holds(blocks, 256))) {
       std::snprintf(name, sizeof(name), "%s_%s", kNames[op], cols ? "cols" : "lanes");
       p.add(name, (uint32_t)(cols ? groups : blocks), 1, !cols ? 256 : op == TILER_HIP_FOLD_MAXIMUM ? 512 : 576)
           .ptr(x).ptr(out).u64(cols ? groups : outputs).u64(contributors).u64(inner).f32(scale).f32(bias);
