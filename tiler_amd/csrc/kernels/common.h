@@ -95,9 +95,14 @@ __device__ __forceinline__ float fold_combine(const FoldRule& r, float acc, floa
 // product before it is rounded, the reference after).  A fold whose result
 // mode flushes with the sign needs nothing more inside its chain, since every
 // result is read next as a flushed operand: only its last result is flushed,
-// by flush_sign.  Called before the first load, so no arithmetic precedes it.
-__device__ __forceinline__ void flush_operands_in_hardware() {
-  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), 2" ::: "memory");
+// by flush_sign.  Returns x advanced by a zero that only the switch produces:
+// what is loaded through the result depends on the switch, so no arithmetic on
+// it can be scheduled ahead (the compiler does not know that the mode changed,
+// and a memory clobber alone orders loads and stores, not adds).
+__device__ __forceinline__ const float* flush_operands_in_hardware(const float* x) {
+  uint64_t none;
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), 2\n\ts_mov_b64 %0, 0" : "=s"(none) : : "memory");
+  return x + none;
 }
 // A subnormal to the zero of its sign, by integer operations (no mode applies).
 __device__ __forceinline__ float flush_sign(float v) {

@@ -516,7 +516,7 @@ __device__ __forceinline__ void staged_rule_dispatch(const float* __restrict__ x
                                                      float* __restrict__ out, const tiler::FoldRule& rule) {
   __shared__ __align__(16) float lds[kRuleStageFloats<R>];
   const bool in = rule.in_mode > 1u, res = rule.out_mode > 1u, hw = tiler::hardware_modes(rule);
-  if (hw) tiler::flush_operands_in_hardware();
+  if (hw) x = tiler::flush_operands_in_hardware(x);
   if constexpr (R <= 16) {  // the relay fold (rows of at least 256 elements per stage)
     if (hw && res) staged_rule_relay_body<R, kVec, true, true, true>(x, nrows, length, out, rule, lds);
     else if (hw) staged_rule_relay_body<R, kVec, true, false, true>(x, nrows, length, out, rule, lds);
@@ -728,7 +728,7 @@ __device__ __forceinline__ void coop_rule_rows(const float* __restrict__ x, uint
                                                const tiler::FoldRule& rule, float* __restrict__ lds) {
   // (a lone contributor is transported, not read by an add: the general rule)
   if (tiler::hardware_modes(rule) && extent > 1) {
-    tiler::flush_operands_in_hardware();
+    x = tiler::flush_operands_in_hardware(x);
     coop_rows<kPacked>(x, rows, extent, participants, chunk, rounds, participant_major, out, rule.out_mode > 1u,
                        [&](float v) { return tiler::fold_contributor_hw(rule, v); },
                        [](float acc, float t) { return acc + t; }, lds);
