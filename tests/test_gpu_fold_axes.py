@@ -27,6 +27,20 @@ def test_adjacent_axes_route(shape, form, variant, name):
     assert rz.symbols == [f"tiler_fold_{name}_f32_{form}"]
 
 
+@pytest.mark.parametrize("shape,variant,symbol", [
+    ((49152, 21), L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"), ((49153, 21), L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    ((49153, 22), L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((262145, 18), L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((262145, 17), L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    ((131072, 17), L.FOLD_FMA, "tiler_fold_fma_f32"), ((131073, 17), L.FOLD_FMA, "tiler_sum_f32_staged_r256_u_m"),
+    ((65536, 23), L.FOLD_FMA, "tiler_fold_fma_f32"), ((65537, 23), L.FOLD_FMA, "tiler_sum_f32_staged_r256_u_m"),
+    ((100, 20), L.FOLD_SQUARED, "tiler_sum_f32_staged_r256_m"), ((100, 17), L.FOLD_SUM, "tiler_sum_f32_staged_r256_u"),
+])
+def test_short_rows(shape, variant, symbol):
+    rz = realize(L.PROGRAM_FOLD, shape, rank=2, grouping=(0b10,), variant=variant, flags=L.REGION_ALIGNED16)
+    assert rz.symbols == [symbol]
+
+
 @pytest.mark.parametrize("shape,mask,symbol", [
     ((4, 8, 64), 0b101, "tiler_fold_sum_f32"),         # not adjacent
     ((2, 5, 300), 0b010, "tiler_fold_sum_f32"),        # too few contributors
@@ -43,8 +57,8 @@ def test_adjacent_axes_are_recognized(shape, mask, symbol):
 
 @pytest.mark.parametrize("shape,mask,variant,symbol", [
     # 2^32 work items and more do not fit a launch: the grid-stride form takes them
-    ((1 << 28, 16), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
-    (((1 << 28) - 16, 16), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
+    ((1 << 28, 24), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
+    (((1 << 28) - 16, 24), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
     ((1 << 26, 257), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),
     (((1 << 26) - 4, 257), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32_rows"),
     ((1 << 24, 2048), 0b10, L.FOLD_MAXIMUM, "tiler_fold_maximum_f32"),

@@ -1535,13 +1535,22 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
     // The reduced axes are adjacent: [outer, contributors, inner].
     char name[48];
     const uint64_t cus = t->compute_units;
+    // Rows of fewer than 24 stay with the general fold where it is faster: many
+    // rows of the maximum, where most of 16 lanes idle (100000 of 18 5.7 us
+    // against 8.2, 1000000 of 16 37.5 / 62.5, but of 24 150 / 63), and few rows
+    // of a prologue off the 4-element grid (33000 of 17 5.3 / 6.1).
+    const bool short_rows =
+        contributors < 24 &&
+        (op == TILER_HIP_FOLD_MAXIMUM ? outputs > 192 * cus && contributors <= (outputs <= 1024 * cus ? 21 : 17)
+                                      : op != TILER_HIP_FOLD_SUM && contributors % 4 != 0 &&
+                                            outputs <= (contributors <= 18 ? 512 : 256) * cus);
     // The maximum's lanes to a row: 16, a wave, or a workgroup for long or few
     // rows.  The sums' staged forms take 64 rows to a workgroup, 256 of fewer
     // than 64 elements (fewer where the rows are few).  More workgroups than a
     // launch holds: the grid-stride form below.
     const uint32_t lanes = contributors >= 2048 || outputs <= 4 * cus ? 256 : contributors > 256 ? 64 : 16;
     const uint32_t per = op == TILER_HIP_FOLD_MAXIMUM ? 256 / lanes : contributors < 64 ? 256 : 64;
-    if (inner == 1 && grid_holds((outputs + per - 1) / per, 256)) {
+    if (inner == 1 && !short_rows && grid_holds((outputs + per - 1) / per, 256)) {
       // contiguous rows: the staged strict sums (a prologue as a rule under
       // the preserving modes), or the maximum's row kernel
       if (op == TILER_HIP_FOLD_SUM) {
