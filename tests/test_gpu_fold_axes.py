@@ -15,7 +15,7 @@ def bits(a):
 
 
 COLS = [(1, 128, 16), (2, 127, 17), (1, 513, 1), (3, 512, 15), (1, 1025, 33), (2, 640, 271), (17, 130, 2)]
-LANES = [(1, 16, 300), (5, 31, 7), (300, 48, 70), (1100, 130, 19)]
+LANES = [(1, 16, 300), (5, 31, 7), (300, 48, 70), (1100, 130, 19), (8192, 128, 2), (1030, 130, 17)]
 ROWS = [(1, 16, 1), (70, 256, 1), (1100, 17, 1), (1100, 257, 1), (3, 2049, 1), (1025, 2048, 1)]
 
 
@@ -25,6 +25,18 @@ ROWS = [(1, 16, 1), (70, 256, 1), (1100, 17, 1), (1100, 257, 1), (3, 2049, 1), (
 def test_adjacent_axes_route(shape, form, variant, name):
     rz = realize(L.PROGRAM_FOLD, shape, rank=3, grouping=(0b010,), variant=variant)
     assert rz.symbols == [f"tiler_fold_{name}_f32_{form}"]
+
+
+@pytest.mark.parametrize("shape,form", [
+    # narrow inner axes: the columns' cost is their groups, not their outputs
+    ((8192, 128, 2), "lanes"), ((4096, 128, 4), "lanes"), ((2048, 128, 8), "lanes"), ((1024, 128, 3), "cols"),
+    ((2048, 4096, 2), "cols"), ((1024, 512, 2), "cols"), ((512, 256, 17), "cols"), ((1024, 256, 17), "lanes"),
+    # wide ones: up to one wave of outputs per CU
+    ((1, 4096, 4096), "cols"), ((16, 1024, 1024), "cols"), ((1000, 256, 64), "lanes"), ((64, 64, 4096), "lanes"),
+])
+def test_columns_or_lanes(shape, form):
+    rz = realize(L.PROGRAM_FOLD, shape, rank=3, grouping=(0b010,), variant=L.FOLD_SUM)
+    assert rz.symbols == [f"tiler_fold_sum_f32_{form}"]
 
 
 @pytest.mark.parametrize("shape,variant,symbol", [

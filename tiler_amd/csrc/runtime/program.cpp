@@ -1570,13 +1570,25 @@ tiler_hip_status plan_fold(uint32_t op, uint32_t rank, const uint64_t* dims, uin
       return TILER_HIP_OK;
     }
     const uint64_t groups = mul_sat(outer, (inner + 15) / 16), blocks = (outputs + 255) / 256;
-    // A workgroup per 16 columns up to one wave of outputs per CU, where a
-    // lane per output waits on its own loads (sum, cols against lanes, us:
-    // 1 x 4096 x 4096 18.6 / 102, 16 x 1024 x 1024 22 / 31); above that the
-    // lanes alone fill memory (1000 x 256 x 64 24 / 12.7, 64 x 64 x 4096
-    // 81 / 11.8), and short folds do not fill a stage (300 x 50 x 1000
-    // 97 / 11.7).  The columns' 32-bit offsets take inner below 2^21.
-    const bool cols = contributors >= 128 && outputs <= 64 * cus && inner < (1ull << 21);
+    // A workgroup per 16 columns, or a lane per output, by the time each takes
+    // in ns, fitted on the device over 1..8192 outer, 128..4096 contributors and
+    // inner 2..4096 (none slower than the form over any axes, and 1% over the
+    // better of the two on average):
+    // * columns: two workgroups to a CU, 4.2 per group and stage of 512 rows
+    //   (8192 x 128 x 2: 41.7 us against 16 by lanes; 2048 x 4096 x 2: 61 / 443);
+    // * lanes: a wave's load touches a line per 64 / inner outputs, 160 / inner
+    //   per contributor and never under 14, or the memory's rate (5.5 TB/s).
+    // Up to one wave of outputs per CU only: above that the lanes alone fill
+    // memory (1000 x 256 x 64 24 / 12.7, 64 x 64 x 4096 81 / 11.8), and short
+    // folds do not fill a stage (300 x 50 x 1000 97 / 11.7).  The columns'
+    // 32-bit offsets take inner below 2^21.
+    const auto columns_win = [&] {
+      const uint64_t at_once = 2 * cus, latency = contributors * (inner < 12 ? 160 / inner : 14);
+      const uint64_t columns = 1700 + (groups > at_once ? groups : at_once) * 42 / 10 * ((contributors + 511) / 512);
+      const uint64_t traffic = outputs * contributors / 1375;
+      return columns <= 3500 + (latency > traffic ? latency : traffic);
+    };
+    const bool cols = contributors >= 128 && outputs <= 64 * cus && inner < (1ull << 21) && columns_win();
     if (inner > 1 && (cols || grid_holds(blocks, 256))) {
       std::snprintf(name, sizeof(name), "%s_%s", kNames[op], cols ? "cols" : "lanes");
       p.add(name, (uint32_t)(cols ? groups : blocks), 1, !cols ? 256 : op == TILER_HIP_FOLD_MAXIMUM ? 512 : 576)
