@@ -588,19 +588,78 @@ tiler_sum_f32_partials_m(const float* __restrict__ x, uint64_t rows, uint64_t ex
 // ascending p and accumulates round totals in ascending r -- the single
 // workgroup tree of tiler-metal's cooperative_workgroup_reduction golden.
 //
-// A participant that folds its cell straight from global memory touches a line
-// per load that its neighbours do not share, and waits for each: 4096 x 4096
-// under the flushing contract took 80 us.  The workgroup instead stages S
-// elements of every cell at a time through LDS (S a power of two that keeps
-// the stage within kCoopFloats), neighbouring participants loading
+// The direct form: a participant folds its cell straight from memory.  Little
+// LDS and few registers, so a CU holds as many workgroups as it has waves for
+// and short cells, bound by a row's latency, overlap (65536 rows of 16
+// participants, 2 rounds of cells of 4: 23 us, 135 staged).
+extern "C" __global__ void __launch_bounds__(1024)
+tiler_sum_f32_cooperative(const float* __restrict__ x, uint64_t extent, uint32_t participants,
+                          uint64_t chunk, uint64_t rounds, uint32_t participant_major,
+                          float* __restrict__ out) {
+  __shared__ float staged[1024];
+  const uint32_t p = threadIdx.x;
+  const float* row = x + (uint64_t)blockIdx.x * extent;
+  float total = -0.0f;
+  for (uint64_t r = 0; r < rounds; ++r) {
+    uint64_t cell = participant_major ? (uint64_t)p * rounds + r : r * participants + p;
+    const float* range = row + cell * chunk;
+    float partial = -0.0f;
+    for (uint64_t w = 0; w < chunk; ++w) partial = partial + range[w];
+    staged[p] = partial;
+    __syncthreads();
+    if (p == 0) {
+      float s = -0.0f;
+      for (uint32_t q = 0; q < participants; ++q) s = s + staged[q];
+      total = total + s;
+    }
+    __syncthreads();
+  }
+  if (p == 0) out[blockIdx.x] = canon(total);
+}
+
+// The same under a FoldRule (evaluate.rs:845-1158 cooperative_grouped_sum_under:
+// every cell, the partials and the round totals seeded at their first value).
+extern "C" __global__ void __launch_bounds__(1024)
+tiler_sum_f32_cooperative_m(const float* __restrict__ x, uint64_t extent, uint32_t participants,
+                                   uint64_t chunk, uint64_t rounds, uint32_t participant_major,
+                                   float* __restrict__ out, tiler::FoldRule rule) {
+  __shared__ float staged[1024];
+  const uint32_t p = threadIdx.x;
+  const float* row = x + (uint64_t)blockIdx.x * extent;
+  float total = 0.0f;
+  for (uint64_t r = 0; r < rounds; ++r) {
+    uint64_t cell = participant_major ? (uint64_t)p * rounds + r : r * participants + p;
+    const float* range = row + cell * chunk;
+    float partial = tiler::fold_contributor(rule, range[0]);
+    for (uint64_t w = 1; w < chunk; ++w)
+      partial = tiler::fold_combine(rule, partial, tiler::fold_contributor(rule, range[w]));
+    staged[p] = partial;
+    __syncthreads();
+    if (p == 0) {
+      float s = staged[0];
+      for (uint32_t q = 1; q < participants; ++q) s = tiler::fold_combine(rule, s, staged[q]);
+      total = r == 0 ? s : tiler::fold_combine(rule, total, s);
+    }
+    __syncthreads();
+  }
+  if (p == 0) out[blockIdx.x] = canon(total);
+}
+
+// The staged forms (*_staged, *_packed), for longer cells and for the modes the
+// hardware applies: a participant that folds its cell straight from memory
+// touches a line per load that its neighbours do not share, and waits for each
+// (4096 x 4096 under the flushing contract took 80 us).  The workgroup instead
+// stages S elements of every cell at a time through LDS (S a power of two that
+// keeps the stage within kCoopFloats), neighbouring participants loading
 // neighbouring elements, and each folds its cell's run from there; the cells
 // lie S + 4 floats apart, so 16 lanes' 16-byte reads touch every bank once.
-// Stages of 20 KiB leave six workgroups to a CU to overlap one's loads with
-// another's fold: 19 us, 3.5 TB/s (1024 x 16384 98 -> 18.5 us).
+// One buffer, with a barrier on both sides of a fold: stages of 20 KiB leave
+// six workgroups to a CU to overlap one's loads with another's fold: 19 us,
+// 3.5 TB/s (1024 x 16384 98 -> 18.5 us).  The planner's rule says where each
+// form is the faster one.
 //
-// combine(acc, t) and contributor(v) are the rule's (evaluate.rs:845-1158
-// cooperative_grouped_sum_under: every cell, the partials and the round totals
-// seeded at their first value); kVec: 16-byte loads.
+// combine(acc, t) and contributor(v) are the rule's, with the same seeds;
+// kVec: 16-byte loads.
 constexpr uint32_t kCoopFloats = 5120;
 
 // The largest power of two S <= 64 with participants * (S + 4) floats in the
@@ -740,15 +799,15 @@ __device__ __forceinline__ void coop_rule_rows(const float* __restrict__ x, uint
 }
 
 extern "C" __global__ void __launch_bounds__(1024)
-tiler_sum_f32_cooperative(const float* __restrict__ x, uint64_t extent, uint32_t participants,
-                          uint64_t chunk, uint64_t rounds, uint32_t participant_major,
-                          float* __restrict__ out) {
+tiler_sum_f32_cooperative_staged(const float* __restrict__ x, uint64_t extent, uint32_t participants,
+                                 uint64_t chunk, uint64_t rounds, uint32_t participant_major,
+                                 float* __restrict__ out) {
   __shared__ __align__(16) float lds[kCoopFloats + 1024];  // the stage, then the partials
   coop_rows<false>(x, gridDim.x, extent, participants, chunk, rounds, participant_major, out, false,
                    [](float v) { return v; }, [](float acc, float t) { return acc + t; }, lds);
 }
 extern "C" __global__ void __launch_bounds__(1024)
-tiler_sum_f32_cooperative_m(const float* __restrict__ x, uint64_t extent, uint32_t participants,
+tiler_sum_f32_cooperative_staged_m(const float* __restrict__ x, uint64_t extent, uint32_t participants,
                             uint64_t chunk, uint64_t rounds, uint32_t participant_major,
                             float* __restrict__ out, tiler::FoldRule rule) {
   __shared__ __align__(16) float lds[kCoopFloats + 1024];

@@ -209,6 +209,47 @@ static void add_serial_fold(const Target& t, uint32_t src, bool src_aligned, uin
 // against one row to a workgroup, us: 65536 rows of 16 participants 14.8 / 130,
 // 4096 of 64 19.0 / 25.8, 30000 of 20 21.6 / 144.
 constexpr uint32_t kCoopPackedThreads = 256;
+// The cooperative sum's forms for cells of c contributors.  Staging pays per
+// cell read, and costs the occupancy its LDS and registers take (six workgroups
+// a CU at most), so short cells and small groups stay direct unless all their
+// rows are resident together; by how dear a combine is (us, staged / direct):
+// * a plain add: packed up to 32 participants or from cells of 16 (65536 rows
+//   of 128 cells of 1: packed 70 / 29).  Staged from cells of 64 (512
+//   rows of 20 x 64 x 8 rounds: 28 / 42), the more participants the more rows
+//   (2048 of 16 x 64 x 8: 68 / 48); above 256 participants with a row to each
+//   CU (4 rows of 512 x 64: 20 / 19); from cells of 16 for 48..256 (8192 of 64
+//   x 16 x 2: 31 / 38; 65536 of 16 x 4 x 2: 135 / 23);
+// * the modes the hardware applies, where the direct form flushes in software:
+//   packed always; staged from 48 participants (65536 of 256 cells of 1: 315 /
+//   1250), fewer only where cells are long or the rows resident (65536 of 4 x 4
+//   x 2: 168 / 38; 512 of 16 x 4 x 8: 14.6 / 30.8);
+// * any other rule (a prologue too), the same arithmetic in all: packed up to 8 participants, to
+//   32 (64 from cells of 16) while cells are at most 64; staged from 48 with a
+//   row to each CU, cells of 64 or resident rows (1024 of 256 x 16 x 2: 57 /
+//   80; 2048 of 256 x 16: 113 / 58).  Fewer rows are within a fifth either way.
+// Measured over 1..1024 participants, cells of 1..256, 1, 2 and 8 rounds, 4 to
+// 65536 rows: none slower than the direct form, and within 1% of the best for
+// the first two.
+enum class CoopForm { kDirect, kStaged, kPacked };
+static CoopForm coop_form(const Target& t, uint64_t rows, uint64_t P, uint64_t c, bool packable,
+                          const FoldRuleHost* rule) {
+  const uint64_t cus = t.compute_units;
+  const bool resident = rows <= 4 * cus;
+  bool packed, staged;
+  if (!rule) {
+    packed = P <= 32 || c >= 16;
+    staged = c >= 64 ? (P <= 256 || rows >= cus) && P >= (!resident ? 32u : rows > 2 * cus ? 20u : 1u)
+                     : c >= 16 && P >= 48 && P <= 256 && rows > cus;
+  } else if (rule->in_mode == 2 && rule->out_mode != 3) {  // tiler::hardware_modes
+    packed = true;
+    staged = resident ? P >= 4 || c >= 16
+                      : P >= 48 || (P >= 32 && c >= 16) || (P >= 20 && c >= 64) || (P >= 16 && c >= 256);
+  } else {
+    packed = P <= 8 || (c <= 64 && (P <= 32 || (c >= 16 && P <= 64)));
+    staged = P >= 48 && rows >= cus && (c >= 64 || (resident && P <= 256));
+  }
+  return packable && packed ? CoopForm::kPacked : staged ? CoopForm::kStaged : CoopForm::kDirect;
+}
 tiler_hip_status plan_sum_f32(const Target& t, uint64_t rows, uint64_t extent,
                               const tiler_hip_sum_plan& sp, const uintptr_t* addr, Program& p,
                               const FoldRuleHost* rule) {
@@ -256,7 +297,9 @@ tiler_hip_status plan_sum_f32(const Target& t, uint64_t rows, uint64_t extent,
       if (P == 0 || P > 1024 || c == 0 || R == 0 || P * c * R != extent)
         return p.refuse(TILER_HIP_REFUSE_INVALID_ARGUMENT, "grouping does not cover the axis exactly");
       if (rows > 0x7fffffffull) return p.refuse(TILER_HIP_REFUSE_CAPACITY, "more rows than the launch grid holds");
-      if (R == 1 && 2 * P <= kCoopPackedThreads && rows >= 8ull * t.compute_units) {
+      const bool packable = R == 1 && 2 * P <= kCoopPackedThreads && rows >= 8ull * t.compute_units;
+      const CoopForm form = coop_form(t, rows, P, c, packable, rule);
+      if (form == CoopForm::kPacked) {
         // many rows of small groups: whole rows packed into a workgroup
         const uint32_t per = (uint32_t)(kCoopPackedThreads / P);
         Launch& l = p.add(rule ? "tiler_sum_f32_cooperative_packed_m" : "tiler_sum_f32_cooperative_packed",
@@ -265,7 +308,10 @@ tiler_hip_status plan_sum_f32(const Target& t, uint64_t rows, uint64_t extent,
         if (rule) l.blob(rule, sizeof(*rule), 4);
         return TILER_HIP_OK;
       }
-      Launch& l = p.add(rule ? "tiler_sum_f32_cooperative_m" : "tiler_sum_f32_cooperative", (uint32_t)rows, 1, (uint32_t)P)
+      const bool staged = form == CoopForm::kStaged;
+      const char* const name = rule ? (staged ? "tiler_sum_f32_cooperative_staged_m" : "tiler_sum_f32_cooperative_m")
+                                    : (staged ? "tiler_sum_f32_cooperative_staged" : "tiler_sum_f32_cooperative");
+      Launch& l = p.add(name, (uint32_t)rows, 1, (uint32_t)P)
                       .ptr(x).u64(extent).u32((uint32_t)P).u64(c).u64(R).u32(sp.participant_major ? 1u : 0u).ptr(out);
       if (rule) l.blob(rule, sizeof(*rule), 4);
       return TILER_HIP_OK;

@@ -71,7 +71,9 @@ const EntryRow kEntries[] = {
     {"tiler_sum_f32_staged_r256_u_m", "serial-sum-f32/serial+rule", 2},
     {"tiler_sum_f32_partials_m", "serial-sum-f32/multipass+rule", 2},
     {"tiler_sum_f32_cooperative_m", "serial-sum-f32/cooperative-workgroup+rule", 2},
-    {"tiler_sum_f32_cooperative_packed", "serial-sum-f32/cooperative-workgroup", 2},
+    {"tiler_sum_f32_cooperative_staged", "strict-serial-sum-f32/cooperative-workgroup", 2},
+    {"tiler_sum_f32_cooperative_staged_m", "serial-sum-f32/cooperative-workgroup+rule", 2},
+    {"tiler_sum_f32_cooperative_packed", "strict-serial-sum-f32/cooperative-workgroup", 2},
     {"tiler_sum_f32_cooperative_packed_m", "serial-sum-f32/cooperative-workgroup+rule", 2},
     {"tiler_fold_f32_m", "serial-sum-f32/serial-any-axes+rule", 2},
     {"tiler_map_f32_m", "pointwise-f32+modes", 3},
