@@ -35,8 +35,10 @@ def test_staged_tiles_keep_the_large_products():
                   (3000, 4096, 4096), (1536, 3000, 3400), (1045, 2536, 2248)):
         rz = realize(L.PROGRAM_CONTRACTION, shape, dtype=L.BF16, permissions=RE)
         assert rz.symbols[0].startswith(("tiler_contract_bf16_t256", "tiler_contract_bf16_t128")), shape
-    rz = realize(L.PROGRAM_CONTRACTION, (3000, 2049, 1024), dtype=L.BF16, permissions=RE)
-    assert rz.symbols == ["tiler_contract_bf16_g128"]
+    # n off the 8-element grid: the general tiles
+    for shape in ((3000, 2049, 1024), (3000, 1001, 512), (4000, 513, 512), (2178, 1278, 1840)):
+        rz = realize(L.PROGRAM_CONTRACTION, shape, dtype=L.BF16, permissions=RE)
+        assert rz.symbols == ["tiler_contract_bf16_g128"], shape
 
 
 def _operands(rng, m, n, k):

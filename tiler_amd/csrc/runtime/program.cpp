@@ -903,9 +903,11 @@ static uint64_t ksplit_grid(uint64_t m, uint64_t n, uint32_t mb, uint32_t nb) {
 //   lines, + 136 per block, the fold of the partial tiles).  The rounds are
 //   those of the XCD with the most panels (1045 x 2536 x 2248 in 6 x 8 tiles:
 //   220 tiles, 33 on some XCDs of 32 CUs, 47 us against 34 staged); two
-//   workgroups of at most 80 KiB share a CU, so a part round costs them less;
-// * 128-tiles: 3400 + 660 per 64-deep k tile, twice that in the general form,
-//   which serves n off the 8-element grid.
+//   workgroups of at most 80 KiB (slots and fold) share a CU, so a part round
+//   costs them less;
+// * 128-tiles: 3400 + 660 per 64-deep k tile; in the general form, which serves
+//   n off the 8-element grid, 2500 + 1150 (3000 x 1001 x 512 12.8 us there, 15.4
+//   in 6 x 8 tiles; 2178 x 1278 x 1840 39.0 / 41.9 in 5 x 4).
 // A k-split tile has to be a tenth faster by these to be taken.  From k = 512
 // on each of eight waves has a chunk of its own.
 static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batches) {
@@ -913,7 +915,7 @@ static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, ui
   const uint64_t cus = t.compute_units;
   const uint64_t t128 = mul_sat(mul_sat((m + 127) / 128, (n + 127) / 128), batches);
   if (t128 > cus) return nullptr;
-  const uint64_t staged = (3400 + 660 * ((k + 63) / 64)) * (n % 8 != 0 ? 2 : 1);
+  const uint64_t steps = (k + 63) / 64, staged = n % 8 != 0 ? 2500 + 1150 * steps : 3400 + 660 * steps;
   const KsplitTile* best = nullptr;
   uint64_t best_ns = staged * 9 / 10;
   for (const KsplitTile& c : kKsplitTiles) {
