@@ -40,6 +40,10 @@ __device__ __forceinline__ void contract_bf16_ksplit_body(const uint16_t* __rest
   constexpr uint32_t kSlot = kLoads * 512u;           // bf16 elements of a wave's slot
   constexpr uint32_t kStage = W * kSlot * 2u, kRed = R * kBlocks * 1024u, kC = MB * 16 * kRow * 2u;
   constexpr uint32_t kBytes = kStage > kRed ? (kStage > kC ? kStage : kC) : (kRed > kC ? kRed : kC);
+  // (6 x 4 blocks fold onto 96 KiB; onto two partial tiles, 80, a workgroup that
+  // has its CU to itself took 8.7 against 8.1 us, 1300 x 1001 x 512.)
+  static_assert(kLoads * W > 80 || kBlocks > 20 || kBytes <= 80 * 1024,
+                "the planner counts on two workgroups of such a tile to a CU");
   __shared__ __attribute__((aligned(1024))) uint16_t smem[kBytes / 2];
   const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t tiles_m = (m + MB * 16 - 1) / (MB * 16), tiles_n = (n + NB * 16 - 1) / (NB * 16);

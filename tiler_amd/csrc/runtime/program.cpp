@@ -921,7 +921,7 @@ static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, ui
   for (const KsplitTile& c : kKsplitTiles) {
     const uint64_t tiles = ksplit_grid(m, n, c.mb, c.nb) * batches;  // whole panel groups
     uint64_t rounds = (tiles + cus - 1) / cus * 1000;                // in thousandths
-    if ((c.mb + c.nb) * c.waves <= 40) {
+    if ((c.mb + c.nb) * c.waves <= 40 && c.mb * c.nb <= 20) {
       rounds = (660 * rounds + 340 * (tiles * 1000 / cus)) / 1000;
       if (rounds < 1000) rounds = 1000;
     }
