@@ -29,6 +29,26 @@ def test_tile_choice(m, n, k, form):
         assert rz.symbols == [f"tiler_contract_bf16_{silu}{form}"]
 
 
+def test_long_k_keeps_the_skinny_form():
+    """From k = 2^24 on, 128 rows leave a buffer's 32-bit offsets: the skinny
+    forms with 64-bit addresses, for the library's choice and on request."""
+    def symbol(m, k, **kw):
+        return realize(L.PROGRAM_CONTRACTION, (m, 40, k), dtype=L.BF16, permissions=RE, **kw).symbols
+    for form in (L.FORM_AUTO, L.FORM_CONTRACT_SKINNY):
+        assert symbol(33, (1 << 24) - 8, form=form) == ["tiler_contract_bf16_skinny3"]
+        assert symbol(33, 1 << 24, form=form) == ["tiler_contract_bf16_skinny3_l"]
+    assert symbol(64, 1 << 24, variant=L.EPILOGUE_SILU) == ["tiler_contract_bf16_silu_skinny4_l"]
+    assert symbol(65, 1 << 24) == ["tiler_contract_bf16_g128"]
+    s = L.contraction_structure("bmk", (2, 16, 1 << 24), "nk", (40, 1 << 24), "bmn")
+    assert realize(L.PROGRAM_CONTRACTION, (), dtype=L.BF16, structure=s, permissions=RE).symbols == \
+        ["tiler_contract_bf16_skinny1_l_b"]
+    # 2^32 work items do not fit a launch: the 128-tiles
+    assert realize(L.PROGRAM_CONTRACTION, (1, (1 << 27) - 256, 8), dtype=L.BF16, permissions=RE).symbols == \
+        ["tiler_contract_bf16_skinny1"]
+    assert not realize(L.PROGRAM_CONTRACTION, (1, 1 << 27, 8), dtype=L.BF16,
+                       permissions=RE).symbols[0].startswith("tiler_contract_bf16_skinny")
+
+
 def test_staged_tiles_keep_the_large_products():
     # the last three: several rounds of 128-tiles, and panels that leave some XCDs a second round
     for shape in ((4096, 4096, 4096), (2048, 4096, 4096), (1000, 2048, 512), (3000, 8192, 1024),
@@ -93,6 +113,35 @@ def test_batched_tiles_are_exact_on_integers(ctx, m, n, k):
         for x in bufs:
             x.free()
     assert np.array_equal(got, oracle.bf16_narrow(want).reshape(want.shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(6, 20, (1 << 24) + 8), (20, 7, 1 << 24), (40, 17, (1 << 24) + 72),
+                                   (50, 3, (1 << 24) + 56)])
+def test_long_k_is_exact_on_integers(ctx, m, n, k):
+    """Operands are nonzero in one element of 4096, so every partial sum stays
+    a binary32 integer; among them the last elements of the last row, which lie
+    past 2^32 bytes of k from the first one's in the larger cases."""
+    rng = np.random.default_rng(m + n)
+    at = np.unique(np.concatenate([rng.integers(0, k, k // 4096), np.arange(k - 9, k), np.arange(9)]))
+    av = rng.integers(-3, 4, (m, at.size)).astype(np.float32)
+    bv = rng.integers(-3, 4, (n, at.size)).astype(np.float32)
+    want = (av.astype(np.float64) @ bv.astype(np.float64).T).astype(np.float32)
+    a, b = np.zeros((m, k), np.uint16), np.zeros((n, k), np.uint16)
+    a[:, at], b[:, at] = oracle.bf16_narrow(av).reshape(av.shape), oracle.bf16_narrow(bv).reshape(bv.shape)
+    s = L.contraction_structure("bmk", (2, m // 2, k), "nk", (n, k), "bmn")
+    da, db, dc = ctx.to_device(a), ctx.to_device(b), ctx.alloc(m * n * 2)
+    try:
+        for call in (lambda: ctx.contract_bf16(da, db, m, n, k, dc),
+                     lambda: ctx.contract(L.BF16, s, da, db, dc, permissions=RE)):
+            ctx.fill_u32(dc, 0x7FC17FC1, m * n * 2 // 4)
+            call()
+            ctx.synchronize()
+            assert np.array_equal(dc.download(np.uint16, (m, n)), oracle.bf16_narrow(want).reshape(m, n))
+    finally:
+        da.free()
+        db.free()
+        dc.free()
 
 
 @pytest.mark.gpu

@@ -2,8 +2,8 @@
 // bf16 contraction with the k loop split over the waves of a workgroup, for
 // the products that leave the 128-tiles' chip idle: m <= 64 (decode shapes,
 // *_skinny{1..4}) and the m of a prompt chunk (*_k{MB}x{NB}).  Any m and n, k
-// a multiple of 8, 16-byte aligned operands; the planner keeps 128 rows of k
-// below 2^32 bytes.
+// a multiple of 8, 16-byte aligned operands; 128 rows of k below 2^32 bytes, or
+// the *_skinny{1..4}_l forms (kLong), whose lanes carry 64-bit addresses.
 //
 // A workgroup owns a tile of 16 MB x 16 NB outputs and each of its W waves the
 // whole tile over its own 64-deep chunks of k (wave w chunks w, w + W, ...).
@@ -29,7 +29,9 @@
 // 512 x 4096 x 4096 45 / 25.
 namespace {
 
-template <int MB, int NB, int W, bool kSilu>
+typedef __attribute__((address_space(1))) void global_void;
+
+template <int MB, int NB, int W, bool kSilu, bool kLong = false>
 __device__ __forceinline__ void contract_bf16_ksplit_body(const uint16_t* __restrict__ a,
                                                           const uint16_t* __restrict__ b, uint32_t m, uint32_t n,
                                                           uint32_t k, uint16_t* __restrict__ c) {
@@ -72,7 +74,24 @@ __device__ __forceinline__ void contract_bf16_ksplit_body(const uint16_t* __rest
   for (uint32_t o = 0; o < 2; ++o)
     vbase[o] = (o * 8u + (lane >> 3)) * k * 2u + ((lane & 7u) ^ (o * 4u + (lane >> 4))) * 16u;
   uint16_t* const slot = smem + wave * kSlot;
+  // kLong: the rows past the last read the last one (never stored) and the
+  // chunks past k read chunk 0 (zeroed below), where a buffer would give zeros.
+  auto row_piece = [&](const uint16_t* panel, uint32_t panel_rows, uint32_t j, uint32_t chunk) {
+    const uint32_t row = j * 8u + (lane >> 3), e = chunk * 64u + ((lane & 7u) ^ ((row >> 1) & 7u)) * 8u;
+    return (global_void*)(panel + (uint64_t)(row < panel_rows ? row : panel_rows - 1u) * k + (e < k ? e : 0u));
+  };
   auto issue = [&](uint32_t chunk) {
+    if constexpr (kLong) {
+#pragma unroll
+      for (int j = 0; j < 2 * NB; ++j)
+        __builtin_amdgcn_global_load_lds(row_piece(b + (uint64_t)n0 * k, cols, j, chunk),
+                                         (lds_void*)(slot + (2 * MB + j) * 512), 16, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 2 * MB; ++j)
+        __builtin_amdgcn_global_load_lds(row_piece(a + (uint64_t)m0 * k, rows, j, chunk),
+                                         (lds_void*)(slot + j * 512), 16, 0, 0);
+      return;
+    }
     const uint32_t at = chunk * 128u;
 #pragma unroll
     for (int j = 0; j < 2 * NB; ++j)
@@ -197,26 +216,33 @@ __device__ __forceinline__ void contract_bf16_ksplit_body(const uint16_t* __rest
 
 }  // namespace
 
-#define TILER_CONTRACT_KSPLIT(NAME, MB, NB, W, SILU)                                                 \
+#define TILER_CONTRACT_KSPLIT(NAME, MB, NB, W, SILU, LONG)                                           \
   extern "C" __global__ void __launch_bounds__(64 * W, (W + 3) / 4)                                   \
       NAME(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint32_t m, uint32_t n,     \
            uint32_t k, uint16_t* __restrict__ c) {                                                    \
-    contract_bf16_ksplit_body<MB, NB, W, SILU>(a, b, m, n, k, c);                                     \
+    contract_bf16_ksplit_body<MB, NB, W, SILU, LONG>(a, b, m, n, k, c);                               \
   }                                                                                                   \
   extern "C" __global__ void __launch_bounds__(64 * W, (W + 3) / 4)                                   \
       NAME##_b(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint32_t m, uint32_t n, \
                uint32_t k, uint16_t* __restrict__ c, tiler_geom::BatchGeometry g) {                   \
     uint64_t oa, ob, oc;                                                                              \
     batch_offsets(g, blockIdx.y, oa, ob, oc);                                                         \
-    contract_bf16_ksplit_body<MB, NB, W, SILU>(a + oa, b + ob, m, n, k, c + oc);                      \
+    contract_bf16_ksplit_body<MB, NB, W, SILU, LONG>(a + oa, b + ob, m, n, k, c + oc);                \
   }
 #define TILER_CONTRACT_KSPLIT_BOTH(FORM, MB, NB, W)                                                   \
-  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_##FORM, MB, NB, W, false)                                 \
-  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_silu_##FORM, MB, NB, W, true)
+  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_##FORM, MB, NB, W, false, false)                          \
+  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_silu_##FORM, MB, NB, W, true, false)
+#define TILER_CONTRACT_KSPLIT_LONG(FORM, MB)                                                          \
+  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_##FORM##_l, MB, 1, 8, false, true)                        \
+  TILER_CONTRACT_KSPLIT(tiler_contract_bf16_silu_##FORM##_l, MB, 1, 8, true, true)
 TILER_CONTRACT_KSPLIT_BOTH(skinny1, 1, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(skinny2, 2, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(skinny3, 3, 1, 8)
 TILER_CONTRACT_KSPLIT_BOTH(skinny4, 4, 1, 8)
+TILER_CONTRACT_KSPLIT_LONG(skinny1, 1)
+TILER_CONTRACT_KSPLIT_LONG(skinny2, 2)
+TILER_CONTRACT_KSPLIT_LONG(skinny3, 3)
+TILER_CONTRACT_KSPLIT_LONG(skinny4, 4)
 TILER_CONTRACT_KSPLIT_BOTH(k2x2, 2, 2, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k2x4, 2, 4, 8)
 TILER_CONTRACT_KSPLIT_BOTH(k3x4, 3, 4, 8)

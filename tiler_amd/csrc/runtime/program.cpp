@@ -879,6 +879,9 @@ struct KsplitTile {
 static const KsplitTile kKsplitTiles[] = {{2, 2, 8}, {2, 4, 8}, {3, 4, 8}, {4, 4, 4},
                                           {5, 4, 8}, {6, 4, 4}, {4, 8, 4}, {6, 8, 4}};
 
+// Below this k a tile's rows (up to 128) lie within a buffer's 32-bit offsets.
+constexpr uint64_t kKsplitBufferK = 1ull << 24;
+
 bool is_ksplit(const char* symbol) {
   const char* k = std::strstr(symbol, "_k");
   return k && k[2] >= '1' && k[2] <= '9';
@@ -911,7 +914,7 @@ static uint64_t ksplit_grid(uint64_t m, uint64_t n, uint32_t mb, uint32_t nb) {
 // A k-split tile has to be a tenth faster by these to be taken.  From k = 512
 // on each of eight waves has a chunk of its own.
 static const KsplitTile* ksplit_tile(const Target& t, uint64_t m, uint64_t n, uint64_t k, uint64_t batches) {
-  if (k < 512 || k >= (1ull << 24)) return nullptr;
+  if (k < 512 || k >= kKsplitBufferK) return nullptr;
   const uint64_t cus = t.compute_units;
   const uint64_t t128 = mul_sat(mul_sat((m + 127) / 128, (n + 127) / 128), batches);
   if (t128 > cus) return nullptr;
@@ -982,15 +985,16 @@ tiler_hip_status plan_contract_bf16(const Target& t, uint64_t m, uint64_t n, uin
   const bool pick = form == TILER_HIP_FORM_AUTO;
   // m <= 64 (decode shapes): B streamed once, one workgroup per 16 columns.
   const bool skinny_ok = m <= 64 && k % 8 == 0 && aligned16(addr[a]) && aligned16(addr[b]) &&
-                         (n + 15) / 16 <= 0x7fffffffull;
+                         grid_holds(ksplit_grid(m, n, 1, 1), 512);
   if (form == TILER_HIP_FORM_CONTRACT_SKINNY && !skinny_ok)
     return p.refuse(TILER_HIP_REFUSE_UNSUPPORTED,
                     "skinny-rows: the skinny form takes m <= 64 and k a multiple of 8, aligned operands");
-  // (k past 2^24: the general form, whose offsets are 64 bits)
-  if (skinny_ok && k < (1ull << 24) && (pick || form == TILER_HIP_FORM_CONTRACT_SKINNY)) {
+  // From kKsplitBufferK on the forms with 64-bit addresses (_l).
+  if (skinny_ok && (pick || form == TILER_HIP_FORM_CONTRACT_SKINNY)) {
     const uint32_t mb = (uint32_t)((m + 15) / 16);
     char name[48];
-    std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u", silu ? "silu_" : "", mb);
+    std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u%s", silu ? "silu_" : "", mb,
+                  k < kKsplitBufferK ? "" : "_l");
     p.add(name, (uint32_t)ksplit_grid(m, n, mb, 1), 1, 512).ptr(a).ptr(b).u32(m32).u32(n32).u32(k32).ptr(c);
     return TILER_HIP_OK;
   }
@@ -1201,12 +1205,13 @@ tiler_hip_status plan_contract_general(const Target& t, uint32_t dtype, const ti
       const bool ab_al = aligned16(addr[l]) && (right_kn || aligned16(addr[r])) && strides8;
       char name[48];
       const KsplitTile* ks = nullptr;
-      if (k % 8 == 0 && k < (1ull << 24) && ab_al) {
+      if (k % 8 == 0 && ab_al) {
         static const KsplitTile kSkinny[] = {{1, 1, 8}, {2, 1, 8}, {3, 1, 8}, {4, 1, 8}};
         ks = m <= 64 ? &kSkinny[(m - 1) / 16] : ksplit_tile(t, m, n, k, batches);
       }
       if (ks) {
-        if (m <= 64) std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u_b", silu ? "silu_" : "", ks->mb);
+        if (m <= 64) std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sskinny%u%s_b", silu ? "silu_" : "", ks->mb,
+                                   k < kKsplitBufferK ? "" : "_l");
         else std::snprintf(name, sizeof(name), "tiler_contract_bf16_%sk%ux%u_b", silu ? "silu_" : "", ks->mb, ks->nb);
         p.add(name, (uint32_t)ksplit_grid(m, n, ks->mb, ks->nb), (uint32_t)batches, 64 * ks->waves)
             .ptr(l).ptr(right_slot).u32(m32).u32(n32).u32(k32).ptr(o).blob(&g, sizeof g, 8);

@@ -337,7 +337,8 @@ const EntryRow kEntries[] = {
       {"tiler_contract_bf16_silu_" K, "tensor-contraction-bf16/cooperative+silu", 3}
     TILER_KSPLIT_ROWS("k2x2"), TILER_KSPLIT_ROWS("k2x4"), TILER_KSPLIT_ROWS("k3x4"),
     TILER_KSPLIT_ROWS("k4x4"), TILER_KSPLIT_ROWS("k5x4"), TILER_KSPLIT_ROWS("k6x4"), TILER_KSPLIT_ROWS("k4x8"),
-    TILER_KSPLIT_ROWS("k6x8"),
+    TILER_KSPLIT_ROWS("k6x8"), TILER_KSPLIT_ROWS("skinny1_l"), TILER_KSPLIT_ROWS("skinny2_l"),
+    TILER_KSPLIT_ROWS("skinny3_l"), TILER_KSPLIT_ROWS("skinny4_l"),
 #undef TILER_KSPLIT_ROWS
     // general index structures: the strict fold (geometry in a constant slot),
     // the batched MFMA forms and the right-operand transpose ahead of them
@@ -350,8 +351,10 @@ const EntryRow kEntries[] = {
       {"tiler_contract_bf16_silu_" K "_b", "tensor-contraction-bf16/cooperative-batched+silu", 3}
     TILER_BATCHED_ROWS("t256"), TILER_BATCHED_ROWS("t128"), TILER_BATCHED_ROWS("skinny1"),
     TILER_BATCHED_ROWS("skinny2"), TILER_BATCHED_ROWS("skinny3"), TILER_BATCHED_ROWS("skinny4"),
-    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"), TILER_BATCHED_ROWS("k2x2"), TILER_BATCHED_ROWS("k2x4"), TILER_BATCHED_ROWS("k3x4"), TILER_BATCHED_ROWS("k4x4"), TILER_BATCHED_ROWS("k5x4"),
-    TILER_BATCHED_ROWS("k6x4"), TILER_BATCHED_ROWS("k4x8"), TILER_BATCHED_ROWS("k6x8"),
+    TILER_BATCHED_ROWS("g128"), TILER_BATCHED_ROWS("g128_k"), TILER_BATCHED_ROWS("k2x2"), TILER_BATCHED_ROWS("k2x4"),
+    TILER_BATCHED_ROWS("k3x4"), TILER_BATCHED_ROWS("k4x4"), TILER_BATCHED_ROWS("k5x4"), TILER_BATCHED_ROWS("k6x4"),
+    TILER_BATCHED_ROWS("k4x8"), TILER_BATCHED_ROWS("k6x8"), TILER_BATCHED_ROWS("skinny1_l"),
+    TILER_BATCHED_ROWS("skinny2_l"), TILER_BATCHED_ROWS("skinny3_l"), TILER_BATCHED_ROWS("skinny4_l"),
 #undef TILER_BATCHED_ROWS
 };
 constexpr uint32_t kEntryCount = sizeof(kEntries) / sizeof(kEntries[0]);
