@@ -208,6 +208,9 @@ int main() {
     }
     // Folds over random axis sets (ranks past the limit, empty and huge extents).
     plan_fold((uint32_t)(r() % 5), frank, fdims, fmask, 0x3f800000u, 0u, nullptr, q[2]);
+    // and with what the adjacent-axes forms are chosen from
+    const uintptr_t faddr[kMaxSlots] = {r() % 2 ? 0u : 4u, 0};
+    plan_fold((uint32_t)(r() % 5), frank, fdims, fmask, 0x3f800000u, 0u, nullptr, q[5], Contract{}, &t, nullptr, faddr);
     // Reindex with signed strides and bases, in and out of the source.
     int64_t sstrides[8];
     for (int d = 0; d < 8; ++d) sstrides[d] = (int64_t)(pick(r) % 2000) - 1000;
@@ -218,7 +221,7 @@ int main() {
     const uintptr_t caddr[kMaxSlots] = {r() % 2 ? 0u : 16u, 0, 0, 0, 0, 0};
     plan_contract_general(t, r() % 2 ? TILER_HIP_F32 : TILER_HIP_BF16, cs, (uint32_t)(r() % 3), r() % 2 == 0, caddr,
                           q[4]);
-    for (int i = 0; i < 5; ++i) {
+    for (int i = 0; i < 6; ++i) {
       check(q[i]);
       planned += q[i].nlaunches;
     }
