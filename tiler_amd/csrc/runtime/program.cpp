@@ -785,9 +785,10 @@ static void declare_live_k(Program& p, uint64_t bound) {
 // Register-blocked strict bf16 tiles of 16·T x 16·T, T x T outputs per thread,
 // T in {1, 2, 4}: the one with the least work on the busiest CU -- rounds of
 // tiles over the CUs x outputs per tile x the time per output step, relative
-// weights 31 : 20 : 18 (T = 1 measured 1.4-1.7 x T = 2 per output step on the
-// 128 x 1024 x 3072 and 128 x 3072 x 1024 cells; T = 4 taken a tenth below
-// T = 2).  Returns T.
+// weights 31 : 20 : 18.  Per output step on a full chip these kernels take 31 :
+// 16.8 : 14.4 (1024 x 3072 x 1024: 405, 220, 188 us); the weights lean towards
+// the smaller tiles, which do better where a round is not full (128 x 1024 x
+// 3072: 105, 170, 458; 128 x 3072 x 1024: 64, 63, 157).  Returns T.
 static uint32_t strict_tile(const Target& t, uint64_t m, uint64_t n) {
   const uint64_t cus = t.compute_units;
   uint32_t best = 1;
