@@ -40,8 +40,9 @@ def test_scratch_across_sizes(ctx):
 
 
 def test_scratch_of_other_streams_and_threads(ctx):
-    """Calls on another stream take scratch of their own; calls from two
-    threads on the context's stream do not interleave over the kept one."""
+    """Calls on another stream take scratch of their own; two threads with a
+    context each run at once, and take turns on a shared one (calls on one
+    context never overlap)."""
     import threading
 
     import tiler_amd
@@ -61,12 +62,15 @@ def test_scratch_of_other_streams_and_threads(ctx):
             for b in bufs:
                 b.free()
             assert np.array_equal(got, oracle.bf16_narrow(want).reshape(want.shape))
-    errors = []
+    errors, turn = [], threading.Lock()
 
     def work(k, n):
         try:
-            for _ in range(8):
-                _check(ctx, 17, k, n)
+            with tiler_amd.Context(0) as own:
+                for _ in range(4):
+                    _check(own, 17, k, n)
+                    with turn:
+                        _check(ctx, 17, k, n)
         except BaseException as e:  # noqa: BLE001 (reported by the main thread)
             errors.append(e)
 

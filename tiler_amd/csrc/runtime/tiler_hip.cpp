@@ -488,9 +488,10 @@ bool capturing(hipStream_t s) {
 // small one (the pool gives memory back at each synchronization, so a call
 // that is waited for pays the allocation again).  The buffer grows in powers
 // of two, the outgrown one freed in stream order behind the calls that use it.
-// The lock is held until the call has enqueued everything, so that calls from
-// two threads cannot interleave their launches over the one buffer.  Other
-// streams and larger requests allocate on the stream for the call alone.
+// Calls on one context must not overlap; the lock, held until the call has
+// enqueued everything, keeps ones that do from interleaving their launches over
+// the one buffer.  Other streams and larger requests allocate on the stream for
+// the call alone.
 constexpr uint64_t kScratchKept = 64ull << 20;
 class CallScratch {
  public:
