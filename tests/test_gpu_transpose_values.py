@@ -83,8 +83,8 @@ def test_scratch_of_other_streams_and_threads(ctx):
 
 
 def test_kept_widening_is_exact(ctx):
-    """Results of 32 MiB and up take the form with ordinary stores."""
-    n = (8 << 20) + 5
+    """Results of 48 MiB and up take the form with ordinary stores."""
+    n = (12 << 20) + 5
     x = np.random.default_rng(3).integers(0, 1 << 16, n).astype(np.uint16)
     dx, dy = ctx.to_device(x), ctx.alloc(4 * n)
     try:
@@ -95,3 +95,27 @@ def test_kept_widening_is_exact(ctx):
         dx.free()
         dy.free()
     assert np.array_equal(got, x.astype(np.uint32) << 16)
+
+
+@pytest.mark.parametrize("n", [(12 << 20) - 4, 12 << 20, (1 << 25) + 3, (1 << 25) + 4])
+def test_kept_maps_are_exact(ctx, n):
+    """The scaling and adding maps one 16-byte chunk below 48 MiB of result (the
+    streaming loop), at 48 and at 128 MiB (ordinary stores; the last with a
+    tail), and one chunk past them (streaming again)."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n).astype(np.float32)
+    z = np.ascontiguousarray(x[::-1])
+    dx, dz, dy = ctx.to_device(x), ctx.to_device(z), ctx.alloc(4 * n + 16)
+    try:
+        for call, want in ((lambda: ctx.map(L.MAP_SCALE_BIAS, L.F32, dx, n, dy, a=0.75, b=-2.0),
+                            x * np.float32(0.75) + np.float32(-2.0)),
+                           (lambda: ctx.map(L.MAP_ADD, L.F32, dx, n, dy, x2=dz), x + z)):
+            ctx.fill_u32(dy, 0x7FC12345, n + 4)
+            call()
+            ctx.synchronize()
+            got = dy.download(np.uint32, (n + 4,))
+            assert np.array_equal(got[:n], want.view(np.uint32))
+            assert (got[n:] == 0x7FC12345).all()
+    finally:
+        for b in (dx, dz, dy):
+            b.free()

@@ -152,12 +152,14 @@ __device__ __forceinline__ uint32_t bf16_pack2_rne(float lo, float hi) {
 // An elementwise result of `bytes` in all: streamed past the caches, or left in
 // them where the next pass over it would find it (the 256 MiB last-level cache
 // holds it beside that pass's own output) and it is large enough for that to
-// matter.  The scaling map's store kept, with the widening's before it, takes a
-// chain over 2^24 elements (widen, scale, softmax, narrow) from 89 to 82 us;
-// alone it is as fast either way up to 128 MiB and slower kept beyond (2^26:
-// 94 against 89 us).  One loop for each kind: in one loop the compiler merges
-// the two stores and drops the hint.
-__device__ __forceinline__ bool keep_in_cache(uint64_t bytes) { return bytes - (32ull << 20) <= (96ull << 20); }
+// matter: 48 to 128 MiB.  A chain that widens, scales, softmaxes and narrows,
+// with the scaling map's and the widening's stores kept, goes from 68.2 to 61.8
+// us at 48 MiB, 86.8 to 80.5 at 64 and 167 to 153 at 128, for 3 to 5% more in a
+// map whose result nobody reads (48 MiB 17.8 / 18.7, 128 MiB 44.7 / 46.7).  At
+// 32 MiB the chain gains as little as the map loses (1.3 and 0.8 of 47 and 13).
+// One loop for each kind: in one loop the compiler merges the two stores and
+// drops the hint.
+__device__ __forceinline__ bool keep_in_cache(uint64_t bytes) { return bytes - (48ull << 20) <= (80ull << 20); }
 template <bool kKeep, typename T>
 __device__ __forceinline__ void store_result(T v, T* p) {
   if constexpr (kKeep) *p = v;

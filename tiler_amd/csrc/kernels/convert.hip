@@ -66,10 +66,10 @@ extern "C" __global__ void __launch_bounds__(256)
 tiler_widen_bf16_f32_v8(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
   widen_v8<false>(x, n8, y);
 }
-// The same with ordinary stores, for results of 32 MiB and up: the pass that
-// reads them next finds what the caches hold, and the widening itself is no
-// slower (2^26 elements 82 against 90 us; 2^22, 16 MiB, 7.4 against 6.2, which
-// is why smaller ones stream).
+// The same with ordinary stores, for results of 48 MiB and up: the pass that
+// reads them next finds what the caches hold (tiler::keep_in_cache), and from
+// 96 MiB on the widening itself is no slower (2^26 elements 82 against 90 us; 48
+// MiB 18.1 / 16.7, repaid by the next pass; 32 MiB 13.6 / 11.7, which is not).
 extern "C" __global__ void __launch_bounds__(256)
 tiler_widen_bf16_f32_v8_c(const u32x4* __restrict__ x, uint64_t n8, f32x4* __restrict__ y) {
   widen_v8<true>(x, n8, y);

@@ -147,7 +147,7 @@ tiler_map_bf16(const uint16_t* __restrict__ x, const uint16_t* __restrict__ x2,
 }
 
 // Vectorized maps: 16 bytes per lane per step (4 f32 or 8 bf16 elements),
-// non-temporal loads and stores (f32 results of 32 to 128 MiB: ordinary stores,
+// non-temporal loads and stores (f32 results of 48 to 128 MiB: ordinary stores,
 // tiler::keep_in_cache), the op and the rank-0 broadcast of x2 fixed at compile
 // time.  Every element sees exactly the scalar kernels' arithmetic.
 // The host uses them on 16-byte-aligned operands for the whole 16-byte chunks

@@ -699,8 +699,8 @@ tiler_hip_status plan_convert(Mode mode, uint32_t direction, uint64_t n, const u
   uint64_t head = aligned16(addr[src]) && aligned16(addr[dst]) ? n / 8 * 8 : 0;
   if (mode == Mode::Realized && head != n) head = 0;
   if (head) {
-    // a widened result of 32 MiB and up is left in the caches for its next pass
-    p.add(narrow ? "tiler_narrow_f32_bf16_v8" : head >= (8ull << 20) ? "tiler_widen_bf16_f32_v8_c" : "tiler_widen_bf16_f32_v8",
+    // a widened result of 48 MiB and up is left in the caches for its next pass
+    p.add(narrow ? "tiler_narrow_f32_bf16_v8" : head >= (12ull << 20) ? "tiler_widen_bf16_f32_v8_c" : "tiler_widen_bf16_f32_v8",
           blocks_capped(head / 8, 8192), 1, 256)
         .ptr(src).u64(head / 8).ptr(dst);
     if (head == n) return TILER_HIP_OK;
