@@ -27,6 +27,16 @@ def test_long_k_keeps_64_bit_addresses():
     assert realize(L.PROGRAM_CONTRACTION, (16, 1 << 20, 1 << 24)).symbols == ["tiler_contract_strict_f32_s16"]
 
 
+@pytest.mark.parametrize("m,n,k,form", [
+    # many rounds, or ragged k: the 64 x 64 tiles; few rounds: 16 rows a workgroup
+    (3000, 4492, 1001, "b64"), (2564, 4492, 161, "b64"), (1500, 4492, 127, "b64"), (3000, 1000, 1001, "b64"),
+    (3000, 4492, 64, "b64"), (1024, 3072, 1024, "b32"), (512, 3072, 1024, "b32"), (2102, 203, 65, "b32"),
+    (1566, 1800, 448, "b32"),
+])
+def test_large_products(m, n, k, form):
+    assert realize(L.PROGRAM_CONTRACTION, (m, n, k)).symbols == [f"tiler_contract_strict_f32_{form}"]
+
+
 def test_wide_n_stays_within_the_grid():
     """2^32 work items along n do not fit a launch; a 64 x 64 tile per 256 threads does."""
     assert realize(L.PROGRAM_CONTRACTION, (17, (1 << 28) - 64, 64)).symbols == ["tiler_contract_strict_f32_b32"]

@@ -808,10 +808,15 @@ static uint32_t strict_tile(const Target& t, uint64_t m, uint64_t n) {
 // * 4 rows while that is at most four workgroups per CU: more waves to hide
 //   the operands' latency (256 x 1024 x 1024, 1024 of them: 19.8 us against
 //   25.9 with twice the rows; 128 x 3072 x 1024, 1536: 30.3 against 26.5).
-// * Then 16 rows or the 64 x 64 tiles, by the work on the busiest CU: rounds x
-//   outputs per workgroup x a weight in quarter units, measured per output
-//   step (1024 x 3072 x 1024, three rounds of 64 x 64: 160 against 179 us;
-//   2048 x 2048 x 1024, four: 218 against 212).
+// * Then 16 rows or the 64 x 64 tiles, by the time of the busiest CU in tenths
+//   of a ns, fitted on the device over m 150..4000, n 60..6000, k 64..3000 (0.2%
+//   over the better of the two): 135 per round and step of k, and a round's
+//   start (more where a last stage is ragged); against 310 per round of tiles
+//   of four times the rows, and two to three rounds' worth that the tiles of a
+//   CU take to overlap, the most where rows a multiple of 64 apart meet in the
+//   same channels.  1024 x 3072 x 1024, 12 rounds of 16 rows or three of tiles:
+//   160 against 179 us; 2048 x 2048 x 1024, 16 or four: 218 / 212; 3000 x 4492 x
+//   1001, 53 or 14: 670 / 508.
 // * The column forms address a tile's 64 rows of k with 32-bit offsets.
 enum class StrictForm { kRows4, kRows16, kTile64 };
 static StrictForm strict_f32_form(const Target& t, uint64_t m, uint64_t n, uint64_t k) {
@@ -820,7 +825,9 @@ static StrictForm strict_f32_form(const Target& t, uint64_t m, uint64_t n, uint6
   if (mul_sat(tn, (m + 3) / 4) <= 4 * cus) return StrictForm::kRows4;
   const uint64_t r16 = (mul_sat(tn, (m + 15) / 16) + cus - 1) / cus;
   const uint64_t r64 = (mul_sat(tn, (m + 63) / 64) + cus - 1) / cus;
-  return mul_sat(r16, 1024 * 76) <= mul_sat(r64, 4096 * 72) + 4096 * 12 ? StrictForm::kRows16 : StrictForm::kTile64;
+  const uint64_t t16 = mul_sat(r16, 135 * k + (k % 64 ? 4000 : 2000));
+  const uint64_t start = (k % 64 == 0 ? 1100 : k % 4 == 0 ? 900 : 700) * k, t64 = mul_sat(r64, 310 * k + 10000);
+  return t16 <= t64 || t16 - t64 <= start ? StrictForm::kRows16 : StrictForm::kTile64;
 }
 
 tiler_hip_status plan_contract_strict_f32(const Target& t, uint64_t m, uint64_t n, uint64_t k, const uintptr_t* addr,
