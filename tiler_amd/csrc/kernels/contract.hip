@@ -185,8 +185,11 @@ __device__ __forceinline__ void contract_strict_blocked_body(const T* __restrict
 // (TM FW rows), the others load.
 //
 // Bound by VALU issue where the chip is full (512 x 3072 x 1024: 70 us, 46 T
-// operations/s; the register-blocked 32 x 32 tiles took 113), else by the
-// latency of a block's operands.  Before and now, us: 17 x 1024 x 1024
+// operations/s; the register-blocked 32 x 32 tiles took 113; 77.6 us over
+// rotating operands), else by the latency of a block's operands: at 128 x 3072
+// x 1024 the SIMDs issue VALU instructions two thirds of the time (14.1 M wave
+// instructions of 4 cycles on 1024 SIMDs in 82 k cycles).  Before and now, us,
+// one set of operands repeated: 17 x 1024 x 1024
 // 29 / 10.2, 128 x 3072 x 1024 49 / 27, 128 x 1024 x 3072 90 / 34,
 // 256 x 1024 x 1024 44 / 17.6, 300 x 3000 x 2000 285 / 111.
 template <int TM, int KB, int W, int FW = W>

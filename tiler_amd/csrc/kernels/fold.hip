@@ -213,7 +213,7 @@ __device__ __forceinline__ void fold_lanes_body(const float* __restrict__ x, flo
 // touch each bank once.  Adjacent 16-column tiles share 128-byte lines: blocks
 // r and r + 8 of each 16 (the same XCD, so the same L2) take neighbours.
 // Bound by the chain of adds, then memory: 1 x 4096 x 4096 (67 MB) takes
-// 18.6 us, 3.6 TB/s, where one lane per output with a load per step took
+// 17.6 us, 3.8 TB/s, where one lane per output with a load per step took
 // 1018 us; 4 byte reads of the stage (one per add and lane) took 46 us.
 constexpr uint32_t kColTile = 16, kColStage = 512, kColLoaders = 512, kColPer = kColStage * kColTile / kColLoaders;
 constexpr uint32_t kColStride = kColStage + 4;

@@ -510,7 +510,8 @@ __device__ __forceinline__ void staged_rule_relay_body(const float* __restrict__
 // pair of flushing dimensions, chosen by a uniform branch.  kHw: the modes the
 // hardware applies (flush_operands_in_hardware), which leaves the chain the
 // preserving fold's one add per element instead of an add, a class test and a
-// select: serial 1024 x 16384 under the flushing contract 243 -> 57 us.
+// select: serial 1024 x 16384 under the flushing contract 238 -> 70 us (the
+// preserving fold 56).
 template <int R, bool kVec>
 __device__ __forceinline__ void staged_rule_dispatch(const float* __restrict__ x, uint64_t nrows, uint64_t length,
                                                      float* __restrict__ out, const tiler::FoldRule& rule) {
@@ -654,9 +655,9 @@ tiler_sum_f32_cooperative_m(const float* __restrict__ x, uint64_t extent, uint32
 // neighbouring elements, and each folds its cell's run from there; the cells
 // lie S + 4 floats apart, so 16 lanes' 16-byte reads touch every bank once.
 // One buffer, with a barrier on both sides of a fold: stages of 20 KiB leave
-// six workgroups to a CU to overlap one's loads with another's fold: 19 us,
-// 3.5 TB/s (1024 x 16384 98 -> 18.5 us).  The planner's rule says where each
-// form is the faster one.
+// six workgroups to a CU to overlap one's loads with another's fold: 18.5 us,
+// 3.6 TB/s (1024 x 16384 103 -> 22.5 us over rotating operands).  The planner's
+// rule says where each form is the faster one.
 //
 // combine(acc, t) and contributor(v) are the rule's, with the same seeds;
 // kVec: 16-byte loads.
